@@ -71,11 +71,16 @@ typedef enum scir_hip_status {
 
 /* ---- arithmetic selection --------------------------------------------- */
 typedef enum scir_hip_precision {
-    /* FP32 arithmetic, any summation order; error within
-     * (K+1) * 2^-23 * sum_k |b_k||x_{n-k}| of the exact sum.  K <= 513 runs
-     * as an FP32 Toeplitz contraction on the matrix cores
-     * (v_mfma_f32_16x16x4_f32, twice the non-packed VALU FMA rate), longer
-     * filters as the direct form with fused multiply-adds on the VALU.  Both
+    /* FP32, any summation order; error within
+     * (K+1) * 2^-23 * sum_k |b_k||x_{n-k}| of the exact sum (plus FP32's
+     * subnormal floor, (K+1) * 2^-149).  Short filters, and K <= 513 on small
+     * batches, run as an FP32 Toeplitz contraction on the matrix cores
+     * (v_mfma_f32_16x16x4_f32, twice the non-packed VALU FMA rate); longer
+     * ones up to K = 2049 as the same contraction with samples and taps split
+     * into two scaled fp16 terms, FP32 accumulation (less error than the FP32
+     * kernels' longer sums; segments whose magnitudes fp16 cannot hold
+     * together take the three bf16 terms of BF16X3), up to K = 6689 as BF16X3
+     * and beyond as the direct form with fused multiply-adds on the VALU.  All
      * recompute any non-finite output from the reference loop's terms, so
      * outputs are non-finite exactly where the reference loop's are. */
     SCIR_HIP_PREC_F32 = 0,
@@ -98,9 +103,10 @@ typedef enum scir_hip_precision {
     /* Toeplitz-block contraction on MFMA with one fp16 product (x and b
      * rounded to fp16), FP32 accumulation.  Reported, not accuracy-bound. */
     SCIR_HIP_PREC_FP16 = 3,
-    /* Fastest of F32 / BF16X3 for the shape (autotuned table when loaded,
-     * else built-in cut-over; F32 for K > 6689, beyond the MFMA kernel's
-     * LDS); never FP16, and FFT32 only when the "auto.fft" key is set.  Either
+    /* Fastest of F32 / BF16X3 for the shape whose error is no larger (F32
+     * below the cut-over of the autotuned table, 130 when none is loaded,
+     * and from K = 288 on large batches; F32 for K > 6689, beyond the MFMA
+     * kernel's LDS); never FP16, and FFT32 only when the "auto.fft" key is set.  Either
      * choice keeps the F32 bound and the reference loop's non-finite
      * outputs, so AUTO is the drop-in default. */
     SCIR_HIP_PREC_AUTO = 4,
@@ -260,7 +266,9 @@ SCIR_HIP_API int scir_hip_filtfilt_f64_cpu(const double *x, int64_t ldx, int64_t
  * same layout as x.  A plan holds the host-built, cost-sorted work list and
  * the device work queue; executing it is one persistent launch.  Executing a
  * plan does not allocate, so it may be captured in a HIP graph.
- * precision: F32 (FP32 direct form), F32_EXACT (the reference loop's order,
+ * precision: F32 (the two fp16 terms of the dense mode, or the FP32 direct
+ * form for batches of short or very long filters), F32_EXACT (the reference
+ * loop's order,
  * bitwise), AUTO (resolved when the plan is made: BF16X3 when the batch's
  * multiply-add weighted tap count reaches the tuned MFMA cut-over and the
  * longest filter fits, F32 otherwise), or BF16X3 / FP16 (the MFMA Toeplitz

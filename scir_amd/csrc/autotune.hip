@@ -81,7 +81,10 @@ TuneChoice tune_lookup(int K, int64_t N)
     if (g_over_direct_loader >= 0) c.direct_loader = g_over_direct_loader;
     if (g_over_direct_seg >= 0) c.direct_seg_tiles = g_over_direct_seg;
     if (g_over_dma_bufs >= 0) c.direct_dma_bufs = g_over_dma_bufs;
-    if (g_over_direct_mfma_strip >= 0) c.direct_mfma_strip = g_over_direct_mfma_strip;
+    if (g_over_direct_mfma_strip >= 0) {
+        c.direct_mfma_strip = g_over_direct_mfma_strip;
+        c.direct_mfma_strip_forced = true;
+    }
     if (g_over_mfma_tiles >= 0) c.mfma_tiles = c.mfma_tiles_fp16 = g_over_mfma_tiles;
     if (g_over_auto_min_k >= 0) c.auto_mfma_min_k = g_over_auto_min_k;
     if (g_over_mfma_segs >= 0) {

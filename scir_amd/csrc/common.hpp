@@ -112,6 +112,11 @@ int fir_fft_dev(const float *x, int64_t ldx, const float *b, int K, int64_t B, i
 int fir_mfma_dev(const float *x, int64_t ldx, const float *b, int K, int64_t B, int64_t N,
                  float *y, int64_t ldy, int precision, bool rev, hipStream_t stream,
                  DeviceState *st);
+// F32 by two fp16 terms (fir_f16x2.hip): whether it takes K taps (its LDS
+// leaves room for two workgroups a CU), and the filter itself.
+bool fir_f16x2_takes(int K);
+int fir_f16x2_dev(const float *x, int64_t ldx, const float *b, int K, int64_t B, int64_t N,
+                  float *y, int64_t ldy, bool rev, hipStream_t stream, DeviceState *st);
 // Partial sums (floats) the allocation-free dL/db entry point holds: 4 MiB.
 constexpr size_t kVjpNoAllocPartials = (size_t)1 << 20;
 // Device address of that entry point's scratch array on the current device.
@@ -134,6 +139,13 @@ int fir_mfma_ragged_occupancy(int precision, size_t lds, int *per_cu);
 int fir_mfma_ragged_launch(const float *x, const float *b, float *y, const MfmaRaggedItem *items,
                            int n_items, unsigned int *counter, int precision, int kmax,
                            size_t lds, int grid, hipStream_t stream);
+
+// The same by two fp16 terms: dynamic LDS bytes and resident workgroups per
+// CU for taps up to kmax, and the launch.
+int fir_f16x2_ragged_occupancy(int kmax, size_t *lds, int *per_cu);
+int fir_f16x2_ragged_launch(const float *x, const float *b, float *y, const MfmaRaggedItem *items,
+                            int n_items, unsigned int *counter, int kmax, size_t lds, int grid,
+                            hipStream_t stream);
 
 TuneChoice tune_lookup(int K, int64_t N);
 RaggedTune ragged_tune_lookup();

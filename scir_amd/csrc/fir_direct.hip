@@ -629,6 +629,69 @@ int fir_direct_dev(const float *x, int64_t ldx, const float *b, int K, int64_t B
               : launch_direct<16, false>(x, ldx, b, K, B, N, y, ldy, rev, stream);
 }
 
+namespace {
+
+// F32 by two fp16 terms (fir_f16x2.hip).
+//   * Above 513 taps, the end of the FP32 matrix-core kernel, always: the VALU
+//     form it replaces is slower at every size ([1, 5000], K = 1023: 21.3 ->
+//     17.0 us; [1024, 65536], K = 1023: 1810 -> 378 us).
+//   * Up to 513 the two cost about staged * (27 + ng) against 5 * outputs * ng
+//     (staged: whole segments; ng: groups of 16 taps), which crosses at K = 97
+//     on long rows ([4096, 65536]: 445 / 509 us at K = 65, 698 / 540 at 129,
+//     1274 / 655 at 255), later where rows fill their segments badly
+//     ([4000, 1000], K = 255: 28 / 43 us), and below 2^25 outputs * ng the
+//     FP32 kernel's shorter start wins ([64, 16384], K = 255: 10.3 / 10.8 us;
+//     at K = 512, 22.1 / 12.7).
+bool takes_f16x2(const TuneChoice &tc, int K, int64_t B, int64_t N)
+{
+    if (tc.direct_loader != 3 || tc.direct_mfma_strip_forced || !fir_f16x2_takes(K)) return false;
+    if (K > kMfmaF32MaxK) return true;
+    const int64_t ng = (K + 14) / 16 + 1;
+    const int64_t seg = N <= 4096 ? 4096 : 8192;
+    const int64_t staged = B * ((N + seg - 1) / seg) * seg;
+    return B * N * ng >= (int64_t)1 << 25 && staged * (27 + ng) < 5 * B * N * ng;
+}
+
+// AUTO chooses between BF16x3 and F32 from its cut-over up.  By two fp16 terms
+// F32 is the faster from there ([4096, 65536], K = 200: 610 against 765 us;
+// [2048, 262144], K = 512: 1830 against 2630), but only from here is its error
+// no larger for any of 34 filters and inputs (relative L2 against BF16x3's:
+// 0.82 on average and 0.95 at most at K = 300, 0.68 and 0.82 at 512; 0.85 and
+// 1.05 at 255, 1.08 and 1.32 at 129), and small batches lose its longer start
+// ([256, 1000], K = 1023: 15 against 20 us).
+constexpr int kF16x2AutoMinK = 288;
+constexpr int64_t kF16x2AutoMinWork = (int64_t)1 << 25;  // outputs * K / 16
+
+bool auto_takes_f16x2(const TuneChoice &tc, int K, int64_t B, int64_t N)
+{
+    return K >= kF16x2AutoMinK && B * N * (K / 16) >= kF16x2AutoMinWork &&
+           takes_f16x2(tc, K, B, N);
+}
+
+// F32 beyond the LDS of two fp16 terms: BF16x3 up to its own limit, with less
+// error than the VALU form's long sums (K = 2048: 2.9e-7 against 7.2e-7) and
+// less time but for the smallest batches ([500, 4000]: 43 against 122 us;
+// [1, 65536]: 55 against 40).
+bool takes_bf16x3(const TuneChoice &tc, int K, int64_t B, int64_t N)
+{
+    return tc.direct_loader == 3 && K > kMfmaF32MaxK && B * N >= (int64_t)1 << 20 &&
+           fir_mfma_takes(SCIR_HIP_PREC_BF16X3, K);
+}
+
+// The F32 mode.
+int fir_f32_dev(const float *x, int64_t ldx, const float *b, int K, int64_t B, int64_t N,
+                float *y, int64_t ldy, bool rev, hipStream_t stream, DeviceState *st)
+{
+    const TuneChoice tc = tune_lookup(K, N);
+    if (takes_f16x2(tc, K, B, N))
+        return fir_f16x2_dev(x, ldx, b, K, B, N, y, ldy, rev, stream, st);
+    if (takes_bf16x3(tc, K, B, N))
+        return fir_mfma_dev(x, ldx, b, K, B, N, y, ldy, SCIR_HIP_PREC_BF16X3, rev, stream, st);
+    return fir_direct_dev(x, ldx, b, K, B, N, y, ldy, false, rev, stream, st);
+}
+
+}  // namespace
+
 // Dense dispatch shared by the host tier, the device tier and the dL/dx
 // adjoint (rev = true: the same filter run back to front).
 int fir_dense_dispatch(const float *x, int64_t ldx, const float *b, int32_t K, int64_t B,
@@ -637,7 +700,7 @@ int fir_dense_dispatch(const float *x, int64_t ldx, const float *b, int32_t K, i
 {
     switch (precision) {
     case SCIR_HIP_PREC_F32:
-        return fir_direct_dev(x, ldx, b, K, B, N, y, ldy, false, rev, stream, st);
+        return fir_f32_dev(x, ldx, b, K, B, N, y, ldy, rev, stream, st);
     case SCIR_HIP_PREC_F32_EXACT:
         return fir_direct_dev(x, ldx, b, K, B, N, y, ldy, true, rev, stream, st);
     case SCIR_HIP_PREC_BF16X3:
@@ -650,9 +713,10 @@ int fir_dense_dispatch(const float *x, int64_t ldx, const float *b, int32_t K, i
         if (tc.auto_fft && K >= tc.auto_fft_min_k && x != y)
             return fir_fft_dev(x, ldx, b, K, B, N, y, ldy, rev, stream, st);
         // BF16x3 MFMA from the cut-over up, while its LDS holds the taps.
-        if (K >= tc.auto_mfma_min_k && fir_mfma_takes(SCIR_HIP_PREC_BF16X3, K))
+        if (K >= tc.auto_mfma_min_k && fir_mfma_takes(SCIR_HIP_PREC_BF16X3, K) &&
+            !auto_takes_f16x2(tc, K, B, N))
             return fir_mfma_dev(x, ldx, b, K, B, N, y, ldy, SCIR_HIP_PREC_BF16X3, rev, stream, st);
-        return fir_direct_dev(x, ldx, b, K, B, N, y, ldy, false, rev, stream, st);
+        return fir_f32_dev(x, ldx, b, K, B, N, y, ldy, rev, stream, st);
     }
     default:
         return fail(SCIR_HIP_ERR_INVALID_ARGUMENT, "unknown precision %d", precision);

@@ -79,6 +79,7 @@ using namespace scir;
 struct scir_hip_ragged_plan_s {
     int device = -1;
     int32_t precision = SCIR_HIP_PREC_F32;
+    bool split = false;  // F32 by two fp16 terms
     int64_t S = 0;
     std::vector<int64_t> offs, boffs;  // host copies (per-signal launches)
     int n_items = 0;
@@ -99,10 +100,31 @@ struct scir_hip_ragged_plan_s {
 
 namespace {
 
-enum RaggedMode { kDirect, kDirectExact, kMfma };
+// F32 by two fp16 terms: for batches whose multiply-add weighted mean K and
+// whose multiply-adds reach these, with taps its LDS holds.  Signals of 256 ..
+// 65536 samples, direct form / two terms: K = 33: 55 / 75 us, 48: 64 / 75, 15
+// .. 90 (mean 63): 80 / 88, 3 .. 127 (mean 85): 110 / 94.  300 signals of 64 ..
+// 2000 samples, K = 3 .. 200 (1.7e7 multiply-adds, under half a segment a
+// signal): 12 / 25; 100 of 1000 .. 5000, 3 .. 700 (0.9e8): 18.5 / 17.8.
+constexpr int kSplitMinMeanK = 80;
+constexpr double kSplitMinMacs = 1.3e8;
+
+bool takes_split(const int64_t *offs, const int64_t *b_offs, int64_t S)
+{
+    int kmean = 0, kmax = 0;
+    int64_t nmean = 0;
+    ragged_batch_stats(offs, b_offs, S, &kmean, &nmean, &kmax);
+    double macs = 0.0;
+    for (int64_t s = 0; s < S; ++s)
+        macs += (double)(offs[s + 1] - offs[s]) * (double)(b_offs[s + 1] - b_offs[s]);
+    return kmean >= kSplitMinMeanK && macs >= kSplitMinMacs && fir_f16x2_takes(kmax);
+}
+
+enum RaggedMode { kDirect, kDirectExact, kMfma, kSplit };
 
 // Kernel family of a precision: the FP32 direct form (f32 / auto, or the
-// reference order with f32_exact) or the MFMA contraction (bf16x3 / fp16).
+// reference order with f32_exact) or the MFMA contraction (bf16x3 / fp16).  A
+// plan of the direct form becomes kSplit by takes_split.
 int ragged_mode(int32_t p, RaggedMode *mode)
 {
     switch (p) {
@@ -147,9 +169,8 @@ int scir_hip_ragged_plan_create(const int64_t *offs, const int64_t *b_offs, int6
             // BF16x3 MFMA when the batch's taps (mean K weighted by
             // multiply-adds) reach the ragged cut-over and its LDS holds the
             // longest filter; the FP32 direct form otherwise.  Both keep the
-            // elementwise FP32 bound.  The ragged F32 kernel is the VALU form,
-            // so its cut-over is lower than the dense one (whose F32 runs on
-            // FP32 MFMA up to K = 257).
+            // elementwise FP32 bound.  F32 on such short filters is the VALU
+            // form, so the cut-over is lower than the dense one.
             int kmean = 0, kmax_all = 0;
             int64_t nmean = 0;
             ragged_batch_stats(offs, b_offs, S, &kmean, &nmean, &kmax_all);
@@ -164,6 +185,8 @@ int scir_hip_ragged_plan_create(const int64_t *offs, const int64_t *b_offs, int6
         }
         RaggedMode mode = kDirect;
         SCIR_TRY(ragged_mode(precision, &mode));
+        if (mode == kDirect && takes_split(offs, b_offs, S)) mode = kSplit;
+        const bool mfma_items = mode == kMfma || mode == kSplit;
         DeviceState *st = nullptr;
         SCIR_TRY(current_device_state(&st));
         const RaggedTune rt = ragged_tune_lookup();
@@ -171,15 +194,19 @@ int scir_hip_ragged_plan_create(const int64_t *offs, const int64_t *b_offs, int6
         std::vector<RaggedItem> items;
         std::vector<MfmaRaggedItem> mitems;
         int kmax = 0;
-        SCIR_TRY(build_ragged_items(offs, b_offs, S, mode == kMfma, rt, &items, &mitems, &kmax));
-        const size_t n_items = mode == kMfma ? mitems.size() : items.size();
+        SCIR_TRY(build_ragged_items(offs, b_offs, S, mfma_items, rt, &items, &mitems, &kmax));
+        const size_t n_items = mfma_items ? mitems.size() : items.size();
 
         size_t lds = 0;
         int per_cu = rt.direct_wg_per_cu;
-        if (mode == kMfma) {
-            SCIR_TRY(fir_mfma_ragged_lds(precision, kmax, &lds));
+        if (mfma_items) {
             int fit = 1;
-            SCIR_TRY(fir_mfma_ragged_occupancy(precision, lds, &fit));
+            if (mode == kSplit) {
+                SCIR_TRY(fir_f16x2_ragged_occupancy(kmax, &lds, &fit));
+            } else {
+                SCIR_TRY(fir_mfma_ragged_lds(precision, kmax, &lds));
+                SCIR_TRY(fir_mfma_ragged_occupancy(precision, lds, &fit));
+            }
             per_cu = rt.mfma_wg_per_cu > 0 ? std::min(rt.mfma_wg_per_cu, fit) : fit;
         } else {
             const int hmax = (std::min(std::max(kmax, 1), kSuper) + 6) & ~3;
@@ -191,6 +218,7 @@ int scir_hip_ragged_plan_create(const int64_t *offs, const int64_t *b_offs, int6
         std::unique_ptr<scir_hip_ragged_plan_s> p(new scir_hip_ragged_plan_s);
         p->device = st->device;
         p->precision = precision;
+        p->split = mode == kSplit;
         p->S = S;
         p->offs.assign(offs, offs + S + 1);
         p->boffs.assign(b_offs, b_offs + S + 1);
@@ -201,7 +229,7 @@ int scir_hip_ragged_plan_create(const int64_t *offs, const int64_t *b_offs, int6
         void *counter = nullptr;
         SCIR_TRY(device_alloc(&counter, sizeof(unsigned int), "ragged plan queue counter"));
         p->counter = static_cast<unsigned int *>(counter);
-        if (mode == kMfma)
+        if (mfma_items)
             SCIR_TRY(upload(mitems, &p->mitems));
         else
             SCIR_TRY(upload(items, &p->items));
@@ -228,6 +256,9 @@ int scir_hip_ragged_plan_execute(scir_hip_ragged_plan plan, const float *x, cons
         hipStream_t s = as_stream(stream);
         hipLaunchKernelGGL(ragged_reset_kernel, dim3(1), dim3(1), 0, s, plan->counter);
         SCIR_TRY(check_launch("ragged_reset_kernel"));
+        if (plan->split)
+            return fir_f16x2_ragged_launch(x, b, y, plan->mitems, plan->n_items, plan->counter,
+                                           plan->kmax, plan->lds, plan->grid, s);
         if (mode == kMfma) {
             DeviceState *st = nullptr;
             SCIR_TRY(current_device_state(&st));
@@ -262,7 +293,10 @@ int scir_hip_ragged_plan_execute_per_signal(scir_hip_ragged_plan plan, const flo
             const int64_t len = plan->offs[i + 1] - plan->offs[i];
             const int K = (int)(plan->boffs[i + 1] - plan->boffs[i]);
             if (len == 0) continue;
-            if (mode == kMfma)
+            if (plan->split)
+                SCIR_TRY(fir_f16x2_dev(x + plan->offs[i], len, b + plan->boffs[i], K, 1, len,
+                                       y + plan->offs[i], len, false, s, st));
+            else if (mode == kMfma)
                 SCIR_TRY(fir_mfma_dev(x + plan->offs[i], len, b + plan->boffs[i], K, 1, len,
                                       y + plan->offs[i], len, plan->precision, false, s, st));
             else

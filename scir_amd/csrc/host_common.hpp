@@ -61,6 +61,7 @@ struct TuneChoice {
     int direct_loader = 3;    // 0: one tile per workgroup, 1: register prefetch, 2: LDS DMA,
                               // 3: F32 mode on FP32 MFMA (K <= 513; otherwise as 2)
     int direct_mfma_strip = 0; // 256-output tiles per wave of loader 3 (0: by K)
+    bool direct_mfma_strip_forced = false;  // set through scir_hip_tune_set: loader 3 only
     int direct_seg_tiles = 4; // tiles per workgroup of the pipelined variants
     int direct_dma_bufs = 2;  // LDS buffers of the DMA loader (tiles in flight + 1), 2..4
     int mfma_tiles = 2;       // 32x32 output tiles per wave, BF16x3 MFMA kernel
