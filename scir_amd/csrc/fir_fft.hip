@@ -9,7 +9,9 @@
 // its real part and the second's in its imaginary part, and entries K-1 ..
 // NF-1 of a circular convolution are the linear convolution's outputs.
 // H = FFT(b zero-padded to NF) / NF comes from fir_fft_spectrum_kernel,
-// launched first on the same stream.
+// launched first on the same stream.  Filters beyond one block of 8192 taps
+// run two blocks a pass in fir_fft_pair_kernel, which keeps the spectrum of
+// the segment before for the second block.
 //
 // The transforms run in LDS: radix-16/32 Stockham passes (natural order in
 // and out), each thread loading R points with stride NF/R, multiplying by
@@ -147,6 +149,7 @@ __device__ __forceinline__ constexpr int store_off(int r)
 //   tq[64 + a], a < NF/64: 2*pi*64a/NF      (coarse; fine * coarse gives any
 //                                            angle 2*pi*m/NF within ~1.5 ulp)
 //   tq[64 + NF/64 + m]:   2*pi*m/(R0*R1)   (the second pass's angles, direct)
+//   then, of four passes, 2*pi*m/(R0*R1*R2) (the third pass's)
 constexpr int kFine = 64;
 template <int NF>
 constexpr int tw_fine_coarse() { return kFine + NF / kFine; }
@@ -219,25 +222,48 @@ __device__ __forceinline__ void fft_pass(float2 *d, const float2 *tq,
 }
 
 template <int LOGN> struct Plan;
-template <> struct Plan<12> { static constexpr int T = 256, R0 = 16, R1 = 16, R2 = 16; };
-template <> struct Plan<13> { static constexpr int T = 256, R0 = 16, R1 = 16, R2 = 32; };
-template <> struct Plan<14> { static constexpr int T = 512, R0 = 16, R1 = 32, R2 = 32; };
+template <> struct Plan<12> { static constexpr int T = 256, R0 = 16, R1 = 16, R2 = 16, R3 = 1; };
+template <> struct Plan<13> { static constexpr int T = 256, R0 = 16, R1 = 16, R2 = 32, R3 = 1; };
+// One workgroup fills a CU's LDS: 16 waves hide more of each other's LDS and
+// memory waits than 8 (512 threads, radices 16, 32, 32), for one more pass:
+// [256, 262144], K = 8192: 621 -> 505 us, K = 4096: 357 -> 328.
+template <> struct Plan<14> { static constexpr int T = 1024, R0 = 16, R1 = 16, R2 = 8, R3 = 8; };
+
+// The passes after the first.  Twiddles: direct tables for the second and, of
+// four passes, the third; the last multiplies the fine and the coarse table's.
+template <int LOGN, bool INV>
+__device__ __forceinline__ void fft_rest(float2 *d, const float2 *tq, int tid)
+{
+    using P = Plan<LOGN>;
+    constexpr int NF = 1 << LOGN, R01 = P::R0 * P::R1;
+    // Opaque: the passes of a forward and an inverse transform form the same
+    // addresses and twiddle indices, which would be kept from one to the other
+    // (the four-pass plan has 128 registers a lane).
+    if (P::R3 > 1) asm volatile("" : "+v"(tid));
+    const float2 *direct = tq + tw_fine_coarse<NF>();
+    fft_pass<NF, P::T, P::R1, P::R0, INV, false, true>(d, direct, nullptr, tid);
+    if constexpr (P::R3 > 1) {
+        fft_pass<NF, P::T, P::R2, R01, INV, false, true>(d, direct + R01, nullptr, tid);
+        fft_pass<NF, P::T, P::R3, R01 * P::R2, INV, false>(d, tq, nullptr, tid);
+    } else {
+        fft_pass<NF, P::T, P::R2, R01, INV, false>(d, tq, nullptr, tid);
+    }
+}
 
 template <int LOGN, bool INV, bool MULH>
 __device__ __forceinline__ void fft(float2 *d, const float2 *tq, const float2 *__restrict__ H,
                                     int tid)
 {
     using P = Plan<LOGN>;
-    constexpr int NF = 1 << LOGN;
-    fft_pass<NF, P::T, P::R0, 1, INV, MULH>(d, tq, H, tid);
-    fft_pass<NF, P::T, P::R1, P::R0, INV, false, true>(d, tq + tw_fine_coarse<NF>(), H, tid);
-    fft_pass<NF, P::T, P::R2, P::R0 * P::R1, INV, false>(d, tq, H, tid);
+    fft_pass<1 << LOGN, P::T, P::R0, 1, INV, MULH>(d, tq, H, tid);
+    fft_rest<LOGN, INV>(d, tq, tid);
 }
 
 template <int LOGN>
 constexpr int tw_entries()
 {
-    return tw_fine_coarse<1 << LOGN>() + Plan<LOGN>::R0 * Plan<LOGN>::R1;
+    using P = Plan<LOGN>;
+    return tw_fine_coarse<1 << LOGN>() + P::R0 * P::R1 + (P::R3 > 1 ? P::R0 * P::R1 * P::R2 : 0);
 }
 
 template <int LOGN>
@@ -247,12 +273,21 @@ constexpr size_t lds_bytes()
     return (size_t)(NF + NF / 32 + tw_entries<LOGN>()) * sizeof(float2);
 }
 
-// H[i] = FFT(b zero-padded)[i] / NF, one workgroup.
+// Taps per block of the FFT path: the largest transform (2^14) keeps at
+// least half of each segment as outputs.  Longer filters are cut into blocks
+// of kFftBlockTaps taps (uniformly partitioned overlap-save): block j, taps
+// b[jP, jP + P), filters the input delayed by jP samples.
+constexpr int kFftBlockTaps = 8192;
+
+// H[i] = FFT(b zero-padded)[i] / NF, one workgroup for each block of taps.
 template <int LOGN>
 __global__ __launch_bounds__(Plan<LOGN>::T) void fir_fft_spectrum_kernel(
     const float *__restrict__ b, int K, const float2 *__restrict__ tq_g, float2 *__restrict__ H)
 {
     constexpr int NF = 1 << LOGN, T = Plan<LOGN>::T;
+    b += (int)blockIdx.x * kFftBlockTaps;
+    K = min(K - (int)blockIdx.x * kFftBlockTaps, kFftBlockTaps);
+    H += (int64_t)blockIdx.x * NF;
     extern __shared__ float2 lds_f2[];
     float2 *d = lds_f2;
     float2 *tq = lds_f2 + NF + NF / 32;
@@ -379,6 +414,153 @@ __global__ __launch_bounds__(Plan<LOGN>::T) void fir_fft_kernel(
     }
 }
 
+// Two blocks of taps in one pass: y_s = IFFT(X_s H0 + X_{s-1} H1) with X_s the
+// transform of the window [8192 (s-1), 8192 (s+1)) of segment s.  A workgroup
+// walks a run of segments of two streams (rows, or runs of one row), which are
+// the real and imaginary parts of one signal.  Each thread keeps the 16 points
+// of X_{s-1} that it multiplies, so a segment costs one transform each way and
+// its outputs are written once; block by block it cost two of each (and a read
+// and a write of y): [256, 262144], K = 16384: 1173 -> 446 us.
+// One workgroup fits a CU (153 KB of LDS), so the transforms' LDS phases and
+// arithmetic alternate; that, not memory, bounds it.
+// A run that does not start its row first transforms the window before it.
+template <bool REV>
+__global__ __launch_bounds__(Plan<14>::T) void fir_fft_pair_kernel(
+    const float *__restrict__ x, int64_t ldx, float *__restrict__ y, int64_t ldy, int64_t N,
+    const float2 *__restrict__ H, const float2 *__restrict__ tq_g, int64_t spr, int64_t run,
+    int64_t runs_per_row, int64_t streams, int accumulate, const float *__restrict__ bfull,
+    int Kfull, int64_t j0, int64_t final_len)
+{
+    using P = Plan<14>;
+    constexpr int NF = 1 << 14, T = P::T, SEG = kFftBlockTaps, M = SEG / T;
+    constexpr int R0 = P::R0, B0 = NF / R0;  // the inverse transform's first pass
+    static_assert(2 * SEG == NF && SEG % T == 0 && B0 == T && T % 32 == 0, "pass shapes");
+    extern __shared__ float2 lds_f2[];
+    float2 *d = lds_f2;
+    float2 *tq = lds_f2 + NF + NF / 32;
+    int tid = threadIdx.x;
+    for (int i = tid; i < tw_entries<14>(); i += T) tq[i] = tq_g[i];
+
+    struct Stream {
+        const float *x;
+        float *y;
+        int64_t seg0, count;  // first segment, segments
+    };
+    auto stream = [&](int64_t u) {
+        if (u >= streams) return Stream{x, y, 0, 0};
+        const int64_t row = u / runs_per_row, s0 = (u - row * runs_per_row) * run;
+        return Stream{x + row * ldx, y + row * ldy, s0, min(run, spr - s0)};
+    };
+    const Stream sa = stream(2 * (int64_t)blockIdx.x), sb = stream(2 * (int64_t)blockIdx.x + 1);
+    const int64_t steps = max(sa.count, sb.count);
+
+    auto lane = [&]() { return (unsigned int)(REV ? T - 1 - tid : tid); };
+    // The window of segment `seg` of one stream, samples tid + T m; zeros
+    // outside the row and past the stream's run.
+    auto load = [&](const Stream &st, int64_t seg, bool wanted, float (&v)[2 * M]) {
+        const int64_t t0 = (seg - 1) * SEG;
+        if (wanted && t0 >= 0 && t0 + NF <= N) {
+            // A uniform base and a 32-bit lane offset.
+#pragma unroll
+            for (int m = 0; m < 2 * M; ++m)
+                v[m] = (REV ? st.x + (N - t0 - T * (m + 1)) : st.x + (t0 + T * m))[lane()];
+        } else {
+#pragma unroll
+            for (int m = 0; m < 2 * M; ++m) {
+                const int64_t t = t0 + tid + T * m;
+                v[m] = 0.0f;
+                if (wanted && t >= 0 && t < N) v[m] = st.x[REV ? N - 1 - t : t];
+            }
+        }
+    };
+    float wa[2 * M], wb[2 * M];
+    auto fill = [&]() {
+#pragma unroll
+        for (int m = 0; m < 2 * M; ++m)
+            d[pad(tid) + m * (T + T / 32)] = make_float2(wa[m], wb[m]);
+        __syncthreads();
+    };
+    float2 prev[R0];  // X_{s-1} at tid + B0 r
+#pragma unroll
+    for (int r = 0; r < R0; ++r) prev[r] = make_float2(0.0f, 0.0f);
+    if (sa.seg0 > 0 || sb.seg0 > 0) {
+        load(sa, sa.seg0 - 1, sa.count > 0, wa);
+        load(sb, sb.seg0 - 1, sb.count > 0, wb);
+        fill();
+        fft<14, false, false>(d, tq, nullptr, tid);
+#pragma unroll
+        for (int r = 0; r < R0; ++r) prev[r] = d[pad(tid) + r * (B0 + B0 / 32)];
+        __syncthreads();
+    }
+    load(sa, sa.seg0, sa.count > 0, wa);
+    load(sb, sb.seg0, sb.count > 0, wb);
+
+    // The rows of the whole filter (for recomputing non-finite outputs): in
+    // REV mode the block's rows start j0 samples into the physical row.
+    const int64_t Nf = N + j0;
+    auto finish = [&](const Stream &st, float v, int64_t t) {
+        if (!__builtin_isfinite(v) && t < final_len)
+            v = direct_output<false>(REV ? st.x - j0 : st.x, Nf, REV, bfull, Kfull, t + j0);
+        return v;
+    };
+    const __amdgpu_buffer_rsrc_t hr = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<float2 *>(H), 0, 2 * NF * (int)sizeof(float2), 0x00020000);
+    for (int64_t i = 0; i < steps; ++i) {
+        asm volatile("" : "+v"(tid));  // as in fft_rest
+        fill();
+        fft<14, false, false>(d, tq, nullptr, tid);
+        {  // the inverse transform's first pass (fft_pass), with the products
+            float2 v[R0];
+#pragma unroll
+            for (int r = 0; r < R0; ++r) {
+                const float2 X = d[pad(tid) + r * (B0 + B0 / 32)];
+                const float2 h0 = __builtin_bit_cast(float2,
+                    __builtin_amdgcn_raw_buffer_load_b64(hr, 8 * tid, 8 * r * B0, 0));
+                const float2 h1 = __builtin_bit_cast(float2,
+                    __builtin_amdgcn_raw_buffer_load_b64(hr, 8 * tid, 8 * (NF + r * B0), 0));
+                v[r] = cadd(cmul(X, h0), cmul(prev[r], h1));
+                prev[r] = X;
+                // Spectra of four points in registers at a time.
+                if (r % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+            }
+            dft<R0, true>(v);
+            __syncthreads();
+            const int bp = pad(tid * R0);
+#pragma unroll
+            for (int r = 0; r < R0; ++r) d[bp + store_off<1, R0>(r)] = v[r];
+            __syncthreads();
+        }
+        fft_rest<14, true>(d, tq, tid);
+        // The next window loads while the outputs go out (no earlier: the
+        // transforms need the registers).
+        load(sa, sa.seg0 + i + 1, i + 1 < sa.count, wa);
+        load(sb, sb.seg0 + i + 1, i + 1 < sb.count, wb);
+        auto store = [&](const Stream &st, bool imag) {
+            if (i >= st.count) return;
+            const int64_t t0 = (st.seg0 + i) * SEG;
+            bool bad = false;
+#pragma unroll
+            for (int m = 0; m < M; ++m) {
+                const float2 o = d[pad(tid) + (m + M) * (T + T / 32)];
+                if (t0 + tid + T * m >= N) break;
+                float out = imag ? o.y : o.x;
+                float &at = (REV ? st.y + (N - t0 - T * (m + 1)) : st.y + (t0 + T * m))[lane()];
+                if (accumulate) out += at;
+                at = out;
+                bad |= !__builtin_isfinite(out);
+            }
+            if (bad)
+                for (int v = tid; v < SEG && t0 + v < N; v += T) {
+                    float &at = st.y[REV ? N - 1 - (t0 + v) : t0 + v];
+                    at = finish(st, at, t0 + v);
+                }
+        };
+        store(sa, false);
+        store(sb, true);
+        __syncthreads();
+    }
+}
+
 // Twiddle tables, one per size, built on first use per device (kept in the
 // device state, freed by scir_hip_shutdown).
 int twiddle_table(DeviceState *st, int logn, hipStream_t s, const float2 **out)
@@ -391,8 +573,12 @@ int twiddle_table(DeviceState *st, int logn, hipStream_t s, const float2 **out)
             cs != hipStreamCaptureStatusNone)
             return fail(SCIR_HIP_ERR_CAPTURE,
                         "the FFT twiddle table is built on first use; run once outside capture");
-        const int r01 = 16 * (logn == 14 ? 32 : 16);  // Plan<logn>::R0 * R1
-        std::vector<float2> h(kFine + NF / kFine + r01);
+        // Direct tables of Plan<logn>: R0 * R1 angles, and R0 * R1 * R2.
+        std::vector<int> direct(1, 256);
+        if (logn == 14) direct.push_back(2048);
+        std::vector<float2> h;
+        h.reserve(kFine + NF / kFine + 2304);
+        h.resize(kFine + NF / kFine);
         for (int i = 0; i < kFine; ++i) {
             const double a = 2.0 * kPi * (double)i / (double)NF;
             h[i] = make_float2((float)std::cos(a), (float)std::sin(a));
@@ -401,10 +587,11 @@ int twiddle_table(DeviceState *st, int logn, hipStream_t s, const float2 **out)
             const double a = 2.0 * kPi * (double)(i * kFine) / (double)NF;
             h[kFine + i] = make_float2((float)std::cos(a), (float)std::sin(a));
         }
-        for (int m = 0; m < r01; ++m) {
-            const double a = 2.0 * kPi * (double)m / (double)r01;
-            h[kFine + NF / kFine + m] = make_float2((float)std::cos(a), (float)std::sin(a));
-        }
+        for (int n : direct)
+            for (int m = 0; m < n; ++m) {
+                const double a = 2.0 * kPi * (double)m / (double)n;
+                h.push_back(make_float2((float)std::cos(a), (float)std::sin(a)));
+            }
         void *p = nullptr;
         SCIR_TRY(device_alloc(&p, h.size() * sizeof(float2), "FFT twiddle table"));
         const hipError_t e = hipMemcpy(p, h.data(), h.size() * sizeof(float2),
@@ -421,6 +608,28 @@ int twiddle_table(DeviceState *st, int logn, hipStream_t s, const float2 **out)
     return SCIR_HIP_OK;
 }
 
+// Spectra of `blocks` blocks of the K taps at b, on stream s: *H (and *tq, the
+// twiddle table) for the filter kernels.
+template <int LOGN>
+int filter_spectra(const float *b, int K, int blocks, hipStream_t s, DeviceState *st,
+                   const float2 **tq, float2 **H)
+{
+    constexpr int NF = 1 << LOGN;
+    constexpr size_t lds = lds_bytes<LOGN>();
+    SCIR_TRY(twiddle_table(st, LOGN, s, tq));
+    StreamScratch &sc = scratch_for(st, s);
+    // The largest size holds two spectra from the start: a filter of more
+    // blocks then needs no more scratch than one of fewer.
+    SCIR_TRY(ensure_scratch(st, sc.fft_spectrum,
+                            (size_t)(LOGN == 14 ? 2 : 1) * NF * sizeof(float2), s));
+    *H = static_cast<float2 *>(sc.fft_spectrum.ptr);
+    SCIR_TRY(allow_dynamic_lds(reinterpret_cast<const void *>(&fir_fft_spectrum_kernel<LOGN>),
+                               (int)lds));
+    hipLaunchKernelGGL((fir_fft_spectrum_kernel<LOGN>), dim3((unsigned)blocks),
+                       dim3(Plan<LOGN>::T), lds, s, b, K, *tq, *H);
+    return check_launch("fir_fft_spectrum_kernel");
+}
+
 template <int LOGN>
 int launch_fft(const float *x, int64_t ldx, const float *b, int K, int64_t B, int64_t N, float *y,
                int64_t ldy, bool rev, bool accumulate, const float *bfull, int Kfull, int64_t j0,
@@ -428,19 +637,13 @@ int launch_fft(const float *x, int64_t ldx, const float *b, int K, int64_t B, in
 {
     constexpr int NF = 1 << LOGN, T = Plan<LOGN>::T;
     const float2 *tq = nullptr;
-    SCIR_TRY(twiddle_table(st, LOGN, s, &tq));
-    StreamScratch &sc = scratch_for(st, s);
-    SCIR_TRY(ensure_scratch(st, sc.fft_spectrum, (size_t)NF * sizeof(float2), s));
-    float2 *H = static_cast<float2 *>(sc.fft_spectrum.ptr);
+    float2 *H = nullptr;
+    SCIR_TRY(filter_spectra<LOGN>(b, K, 1, s, st, &tq, &H));
     constexpr size_t lds = lds_bytes<LOGN>();
     SCIR_TRY(allow_dynamic_lds(reinterpret_cast<const void *>(&fir_fft_kernel<LOGN, false>),
                                (int)lds));
     SCIR_TRY(allow_dynamic_lds(reinterpret_cast<const void *>(&fir_fft_kernel<LOGN, true>),
                                (int)lds));
-    SCIR_TRY(allow_dynamic_lds(reinterpret_cast<const void *>(&fir_fft_spectrum_kernel<LOGN>),
-                               (int)lds));
-    hipLaunchKernelGGL((fir_fft_spectrum_kernel<LOGN>), dim3(1), dim3(T), lds, s, b, K, tq, H);
-    SCIR_TRY(check_launch("fir_fft_spectrum_kernel"));
     const int64_t V = NF - K + 1;
     const int64_t spr = (N + V - 1) / V;
     const int64_t nseg = B * spr;
@@ -456,13 +659,6 @@ int launch_fft(const float *x, int64_t ldx, const float *b, int K, int64_t B, in
                            final_len);
     return check_launch("fir_fft_kernel");
 }
-
-// Taps per block of the FFT path: the largest transform (2^14) keeps at
-// least half of each segment as outputs.  Longer filters are cut into blocks
-// of kFftBlockTaps taps (uniformly partitioned overlap-save): block j, taps
-// b[jP, jP + P), filters the input delayed by jP samples, and its outputs are
-// added to those of the blocks before it.
-constexpr int kFftBlockTaps = 8192;
 
 // FFT size for K taps: the smallest of 2^12, 2^13, 2^14 with NF >= 4K
 // (outputs per segment >= 3/4 NF), else 2^14.
@@ -488,6 +684,44 @@ int fft_block(const float *x, int64_t ldx, const float *b, int K, int64_t B, int
 #undef SCIR_FFT_BLOCK
 }
 
+// Two blocks of taps (K of them at b, more than kFftPairMinTaps) in one pass.
+constexpr int kFftPairMinTaps = 7168;
+
+int fft_block_pair(const float *x, int64_t ldx, const float *b, int K, int64_t B, int64_t N,
+                   float *y, int64_t ldy, bool rev, bool accumulate, const float *bfull,
+                   int Kfull, int64_t j0, int64_t final_len, hipStream_t s, DeviceState *st)
+{
+    const float2 *tq = nullptr;
+    float2 *H = nullptr;
+    SCIR_TRY(filter_spectra<14>(b, K, 2, s, st, &tq, &H));
+    constexpr size_t lds = lds_bytes<14>();
+    const int64_t spr = (N + kFftBlockTaps - 1) / kFftBlockTaps;
+    // Runs per row: the fewest rounds of workgroups over the CUs times a run's
+    // cost (its segments, and half of one for the window before it).
+    const int64_t cus = std::max(1, st->cu_count);
+    int64_t runs = 1;
+    double best = 1e30;
+    for (int64_t c = 1; c <= spr && c <= 4 * cus; ++c) {
+        const int64_t len = (spr + c - 1) / c, n = (spr + len - 1) / len;
+        const int64_t rounds = ((B * n + 1) / 2 + cus - 1) / cus;
+        const double cost = (double)rounds * ((double)len + (n > 1 ? 0.5 : 0.0));
+        if (cost < best) {
+            best = cost;
+            runs = n;
+        }
+    }
+    const int64_t run = (spr + runs - 1) / runs;
+    runs = (spr + run - 1) / run;
+    const int64_t blocks = (B * runs + 1) / 2;
+    if (blocks > 0x7fffffff) return fail(SCIR_HIP_ERR_INVALID_ARGUMENT, "batch too large");
+    auto *kernel = rev ? &fir_fft_pair_kernel<true> : &fir_fft_pair_kernel<false>;
+    SCIR_TRY(allow_dynamic_lds(reinterpret_cast<const void *>(kernel), (int)lds));
+    hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(Plan<14>::T), lds, s, x, ldx, y, ldy,
+                       N, H, tq, spr, run, runs, B * runs, accumulate ? 1 : 0, bfull, Kfull, j0,
+                       final_len);
+    return check_launch("fir_fft_pair_kernel");
+}
+
 }  // namespace
 
 int fir_fft_dev(const float *x, int64_t ldx, const float *b, int K, int64_t B, int64_t N, float *y,
@@ -499,18 +733,23 @@ int fir_fft_dev(const float *x, int64_t ldx, const float *b, int K, int64_t B, i
     if (x == y)
         return fail(SCIR_HIP_ERR_INVALID_ARGUMENT, "the FFT path does not filter in place");
     if (B == 0 || N == 0) return SCIR_HIP_OK;
-    for (int64_t j0 = 0; j0 < K && j0 < N; j0 += kFftBlockTaps) {
-        const int Kj = (int)std::min<int64_t>(kFftBlockTaps, K - j0);
+    for (int64_t j0 = 0, step; j0 < K && j0 < N; j0 += step) {
+        // Two blocks at once, also when the second has no taps but the first
+        // leaves fft_block few outputs a segment ([256, 262144], K = 8192: 505
+        // us by fft_block, 446 by the pair; they cross at about 7100).
+        const bool pair = K - j0 > kFftPairMinTaps && N - j0 > kFftBlockTaps;
+        step = pair ? 2 * kFftBlockTaps : kFftBlockTaps;
+        const int Kj = (int)std::min<int64_t>(step, K - j0);
         // Forward: y[j0 + i] += sum_k b[j0 + k] x[i - k] for i < N - j0.  Back
         // to front the same sums read x from sample j0 on and write y from 0.
         const float *xs = rev ? x + j0 : x;
         float *ys = rev ? y : y + j0;
-        // Block j writes outputs j0 .. j0 + kFftBlockTaps - 1 last (all the
-        // rest when it is the final block).
-        const bool last = j0 + kFftBlockTaps >= K || j0 + kFftBlockTaps >= N;
-        const int64_t final_len = last ? N - j0 : (int64_t)kFftBlockTaps;
-        SCIR_TRY(fft_block(xs, ldx, b + j0, Kj, B, N - j0, ys, ldy, rev, j0 > 0, b, K, j0,
-                           final_len, stream, st));
+        // This pass writes outputs j0 .. j0 + step - 1 last (all the rest when
+        // it is the final one).
+        const bool last = j0 + step >= K || j0 + step >= N;
+        const int64_t final_len = last ? N - j0 : step;
+        SCIR_TRY((pair ? fft_block_pair : fft_block)(xs, ldx, b + j0, Kj, B, N - j0, ys, ldy, rev,
+                                                     j0 > 0, b, K, j0, final_len, stream, st));
     }
     return SCIR_HIP_OK;
 }

@@ -129,3 +129,20 @@ def test_fft_refusals():
     # K = 0 gives zeros like every path
     y = device.fir(torch.ones((2, 50), device="cuda:0"), torch.zeros(0, device="cuda:0"), "fft32")
     assert float(y.abs().max()) == 0.0
+
+
+@pytest.mark.parametrize("B,N,K", [(300, 66000, 16384), (257, 40000, 9000), (3, 8193, 7169),
+                                   (2, 16385, 24577)])
+def test_fft_block_pairs(B, N, K):
+    """Two blocks of taps a pass: runs of several segments that start inside
+    their rows (300 and 257 rows), an odd number of runs, the shortest filter
+    and row it takes, and a second pass that adds to the first."""
+    print(f"fft pairs B={B} N={N} K={K}", flush=True)
+    rng = np.random.default_rng(B + K)
+    x = rng.standard_normal((B, N)).astype(np.float32)
+    b = (rng.standard_normal(K) / np.sqrt(K)).astype(np.float32)
+    xt, bt = torch.tensor(x, device="cuda:0"), torch.tensor(b, device="cuda:0")
+    rows = sorted({0, 1, B // 2, B - 2, B - 1})
+    _check(device.fir(xt, bt, "fft32").cpu().numpy()[rows], x[rows], b)
+    dx = device.vjp_dx(xt, bt, "fft32").cpu().numpy()[rows]
+    _check(np.ascontiguousarray(dx[:, ::-1]), np.ascontiguousarray(x[rows][:, ::-1]), b)
