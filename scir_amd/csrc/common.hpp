@@ -78,6 +78,9 @@ int device_alloc(void **ptr, size_t bytes, const char *what);
 // growing frees the old block.
 int ensure_buffer(DeviceBuffer &buf, size_t bytes, hipStream_t stream);
 
+// Whether `stream` is being captured into a graph.
+bool stream_capturing(hipStream_t stream);
+
 // Makes the scratch block `buf` of device state `st` hold at least `bytes`.
 // A HIP graph captured earlier may hold the old block's address, so growing
 // retires it (freed at scir_hip_shutdown) instead of freeing it; sizes grow

@@ -78,11 +78,16 @@ int device_alloc(void **ptr, size_t bytes, const char *what)
     return SCIR_HIP_OK;
 }
 
-static int refuse_growth_in_capture(size_t bytes, hipStream_t stream)
+bool stream_capturing(hipStream_t stream)
 {
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    if (stream != nullptr && hipStreamIsCapturing(stream, &cs) == hipSuccess &&
-        cs != hipStreamCaptureStatusNone)
+    return stream != nullptr && hipStreamIsCapturing(stream, &cs) == hipSuccess &&
+           cs != hipStreamCaptureStatusNone;
+}
+
+static int refuse_growth_in_capture(size_t bytes, hipStream_t stream)
+{
+    if (stream_capturing(stream))
         return fail(SCIR_HIP_ERR_CAPTURE,
                     "scratch must grow to %zu bytes during stream capture; run the call "
                     "once outside capture first", bytes);

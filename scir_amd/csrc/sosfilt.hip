@@ -27,8 +27,13 @@
 //   1. sos_wave_kernel<STATE>: each chunk's end state from zero state,
 //   2. sos_scan_kernel: per row, z_c = A^L z_{c-1} + e_{c-1},
 //   3. sos_wave_kernel<RUN>: each chunk from z_c.
-// sos_setup_kernel computes C, (A^16)^(2^k) and A^L first.  The first 16
-// outputs of every chunk run from its exact start state (the reference's
+// sos_setup_kernel computes C, (A^16)^(2^k) and A^L first.  Up to 128 chunks
+// a row and four sections the states take no launch of their own: each RUN
+// wave collects its chunk's start state from the end states (collect_state,
+// with the powers of A^L from sos_prepare_kernel), and a filtfilt's first RUN
+// also runs its outputs back to front from zero state (BACK), which gives
+// the second direction's end states without another pass over y.  The first
+// 16 outputs of every chunk run from its exact start state (the reference's
 // arithmetic, bit for bit in chunk 0); the others carry the rounding of the
 // joins (measured ~1e-15 relative).  SCIR_HIP_SOS_REFERENCE_ORDER, and rows
 // of at most 1024 samples, use sos_row_kernel instead: one lane a row, the
@@ -46,7 +51,7 @@ constexpr int kStep = 64 * kGroup;     // samples a wave filters per step
 constexpr int kMaxSections = 16;       // SCIR_HIP_SOS_MAX_SECTIONS
 constexpr int kPowers = 6;             // (A^16)^(2^k), k < 6: lane offsets 1..32
 
-enum { kState = 0, kRun = 1 };
+enum { kState = 0, kRun = 1, kCollect = 2 };
 
 // Kernels are built for S = 1..8 sections exactly (SMAX == S, no run-time
 // guards in the sample loop) and for 9..16 with SMAX = 16 and guards.
@@ -186,6 +191,84 @@ __device__ __forceinline__ void wave_sync()
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// The matrices of the collecting kernels, S sections exactly: C and P as
+// above, then T^(2^k), k < kChunkPowers, T = A^L, and M^(2^k), k < kPowers,
+// M = A^kStep.
+constexpr int kCollectMaxS = 4;
+constexpr int64_t kMaxChunks = 128;  // collected two per lane
+constexpr int kChunkPowers = 7;      // T^64 joins the two halves
+constexpr int64_t kMaxSteps = 64;    // of a chunk: one lane each
+__host__ __device__ constexpr int64_t mats_m(int D)
+{
+    return mats_t(D) + (int64_t)kChunkPowers * D * D;
+}
+__host__ __device__ constexpr int64_t collect_mats_size(int D)
+{
+    return mats_m(D) + (int64_t)kPowers * D * D;
+}
+
+// One wave, a lane per matrix element: the products follow each other with
+// no barrier between (~1/3 of sos_setup_kernel's time at L = 2048, with 13
+// more matrices).  q = L/16.
+template <int S>
+__global__ __launch_bounds__(64) void sos_prepare_kernel(const double *__restrict__ sos, int64_t q,
+                                                         double *__restrict__ mats)
+{
+    constexpr int D = 2 * S;
+    static_assert(D * D <= 64, "one lane per matrix element");
+    __shared__ double base[D][D], res[D][D];
+    const int lane = threadIdx.x;
+    if (lane < D) {
+        // 16 zero-input steps from unit state `lane`: C's column and A^16's
+        Coefs<S> cf;
+        load_coefs(cf, sos, S);
+        double s1[S], s2[S];
+#pragma unroll
+        for (int i = 0; i < S; ++i) {
+            s1[i] = (2 * i == lane) ? 1.0 : 0.0;
+            s2[i] = (2 * i + 1 == lane) ? 1.0 : 0.0;
+        }
+        for (int k = 0; k < kGroup; ++k) mats[k * D + lane] = df2t_step<S>(0.0, s1, s2, cf, S);
+#pragma unroll
+        for (int i = 0; i < S; ++i) {
+            base[2 * i][lane] = s1[i];
+            base[2 * i + 1][lane] = s2[i];
+        }
+    }
+    const bool on = lane < D * D;
+    const int i = on ? lane / D : 0, j = on ? lane % D : 0;
+    if (on) res[i][j] = i == j ? 1.0 : 0.0;
+    wave_sync();
+    // base runs through (A^16)^(2^k); res collects T = (A^16)^q bit by bit.
+    for (int k = 0; k < 2 * kPowers || (q >> k) > 0; ++k) {
+        const double v = base[i][j];
+        if (on && k < 2 * kPowers)
+            mats[(k < kPowers ? mats_p(D) + k * D * D : mats_m(D) + (k - kPowers) * D * D) + lane] =
+                v;
+        double pr = 0.0, sq = 0.0;
+#pragma unroll
+        for (int m = 0; m < D; ++m) {
+            pr = fma(res[i][m], base[m][j], pr);
+            sq = fma(base[i][m], base[m][j], sq);
+        }
+        wave_sync();
+        if (on) {
+            if ((q >> k) & 1) res[i][j] = pr;
+            base[i][j] = sq;
+        }
+        wave_sync();
+    }
+    for (int k = 0; k < kChunkPowers; ++k) {
+        if (on) mats[mats_t(D) + k * D * D + lane] = res[i][j];
+        double sq = 0.0;
+#pragma unroll
+        for (int m = 0; m < D; ++m) sq = fma(res[i][m], res[m][j], sq);
+        wave_sync();
+        if (on) res[i][j] = sq;
+        wave_sync();
+    }
+}
+
 // Inclusive scan over the wave of the lanes' end states: lane l ends with
 // sum_{j <= l} (A^16)^(l-j) e_j.
 template <int D>
@@ -245,16 +328,102 @@ __device__ __forceinline__ void group_span(int64_t gidx, int64_t ngroups, int64_
     }
 }
 
+// A lane's group from zero state, in time order: outputs in place of the
+// samples, end state in s1, s2.
+template <int SMAX, bool REV>
+__device__ __forceinline__ void filter_group(double (&v)[kGroup], int64_t cnt, bool all_full,
+                                             double (&s1)[SMAX], double (&s2)[SMAX],
+                                             const Coefs<SMAX> &cf, int S)
+{
+#pragma unroll
+    for (int i = 0; i < SMAX; ++i) s1[i] = s2[i] = 0.0;
+    if (all_full) {
+        if (!REV) {
+#pragma unroll
+            for (int k = 0; k < kGroup; ++k) v[k] = df2t_step<SMAX>(v[k], s1, s2, cf, S);
+        } else {
+#pragma unroll
+            for (int k = kGroup - 1; k >= 0; --k) v[k] = df2t_step<SMAX>(v[k], s1, s2, cf, S);
+        }
+    } else {
+        if (!REV) {
+#pragma unroll
+            for (int k = 0; k < kGroup; ++k)
+                if (k < cnt) v[k] = df2t_step<SMAX>(v[k], s1, s2, cf, S);
+        } else {
+#pragma unroll
+            for (int k = kGroup - 1; k >= 0; --k)
+                if (k < cnt) v[k] = df2t_step<SMAX>(v[k], s1, s2, cf, S);
+        }
+    }
+}
+
+// w += M u
+template <int D>
+__device__ __forceinline__ void mat_add(double (&w)[D], const double *__restrict__ m,
+                                        const double (&u)[D])
+{
+#pragma unroll
+    for (int i = 0; i < D; ++i)
+#pragma unroll
+        for (int k = 0; k < D; ++k) w[i] = fma(m[i * D + k], u[k], w[i]);
+}
+
+// Lane 0: the sum of M^l e_l over the wave's lanes, M^(2^k) at m[k].  A power
+// is applied only to the `count` states that are there: it may overflow (an
+// unstable filter), and times a zero would be a NaN.
+template <int D>
+__device__ __forceinline__ void reduce_down(double (&e)[D], const double *__restrict__ m, int lane,
+                                            int64_t count)
+{
+#pragma unroll 1
+    for (int k = 0; k < 6; ++k) {
+        double w[D];
+#pragma unroll
+        for (int i = 0; i < D; ++i) w[i] = __shfl_down(e[i], 1 << k, 64);
+        if (lane + (1 << k) < count) mat_add<D>(e, m + k * D * D, w);
+    }
+}
+
+// Chunk c's start state, the same in every lane, from the end states of the
+// row's earlier chunks at zr[chunk*D]: z = sum_j T^(c-1-j) e_j.
+template <int D>
+__device__ __forceinline__ void collect_state(double (&z)[D], const double *zr, int64_t c,
+                                              const double *__restrict__ tp, int lane)
+{
+    double e0[D], e1[D];  // chunk c-1-lane, chunk c-65-lane
+#pragma unroll
+    for (int i = 0; i < D; ++i) {
+        e0[i] = lane < c ? zr[(c - 1 - lane) * D + i] : 0.0;
+        e1[i] = lane + 64 < c ? zr[(c - 65 - lane) * D + i] : 0.0;
+    }
+    reduce_down<D>(e0, tp, lane, std::min<int64_t>(c, 64));
+    if (c > 64) {
+        reduce_down<D>(e1, tp, lane, c - 64);
+        mat_add<D>(e0, tp + 6 * D * D, e1);
+    }
+#pragma unroll
+    for (int i = 0; i < D; ++i) z[i] = __shfl(e0[i], 0, 64);
+}
+
 // One wave per chunk (see the top of the file).  MODE kState: chunks
 // 0..nC-2 of every row from zero state, end states to zs[(row*nC + c)*2S].
 // MODE kRun: every chunk from zs[...] (zero when zs is null), outputs to y.
+// MODE kCollect: kRun with zs as kState left it; BACK also writes the end
+// states, from zero state, of the outputs filtered back to front to
+// zs[rows*nC*2S + ...].  Bound by HBM (a RUN over 32 rows of 262144 moves
+// 134 MB in 27 us, the rate of a large copy) and, on short rows, by the
+// launches: butter(4) there as filtfilt 112 -> 86 us, as sosfilt 55 -> 48,
+// 64 rows of 9000 50 -> 31 and 25 -> 18.  The plan starts 4 waves a SIMD in
+// one go, so the collecting kernels are held to the 128 registers that
+// lets all of them run at once (four sections would spill).
 // REV runs each row back to front; chunk c is c-th in time, and back to
 // front the short chunk (when L does not divide N) comes first, so every
 // chunk starts at a multiple of L (16-byte aligned groups) and only the
 // first group in time can be short; every chunk after the first in time is
 // L long, so A^L is its transition.
-template <int SMAX, int MODE, bool REV>
-__global__ __launch_bounds__(kThreads) void sos_wave_kernel(
+template <int SMAX, int MODE, bool REV, bool BACK = false>
+__global__ __launch_bounds__(kThreads, MODE == kCollect && SMAX <= 3 ? 4 : 1) void sos_wave_kernel(
     const double *x, int64_t ldx, double *y, int64_t ldy, int64_t rows, int64_t N,
     const double *__restrict__ sos, int S, int64_t L, int64_t nC,
     const double *__restrict__ mats, double *__restrict__ zs, int vec)
@@ -277,13 +446,18 @@ __global__ __launch_bounds__(kThreads) void sos_wave_kernel(
     Coefs<SMAX> cf;
     load_coefs(cf, sos, S);
     double zin[D];  // the wave's state at the start of the step (same in every lane)
+    if (MODE == kCollect) {
+        collect_state<D>(zin, zs + row * nC * D, c, mats + mats_t(D), lane);
+    } else {
 #pragma unroll
-    for (int i = 0; i < D; ++i)
-        zin[i] = (MODE == kRun && zs != nullptr && i < d) ? zs[(row * nC + c) * d + i] : 0.0;
+        for (int i = 0; i < D; ++i)
+            zin[i] = (MODE == kRun && zs != nullptr && i < d) ? zs[(row * nC + c) * d + i] : 0.0;
+    }
+    double back[D] = {};  // step `lane` back to front: its end state from zero state
     // x and y may be the same array (filtfilt's second pass runs in place):
     // a step's samples are all read before any is written.
     const double *xr = x + row * ldx;
-    double *yr = (MODE == kRun) ? y + row * ldy : nullptr;
+    double *yr = (MODE != kState) ? y + row * ldy : nullptr;
     const bool vb = vec != 0;
     double *tile = tiles[threadIdx.x >> 6];
     // A step whose 64 groups are all whole covers 8 KB of contiguous memory:
@@ -333,29 +507,8 @@ __global__ __launch_bounds__(kThreads) void sos_wave_kernel(
         } else {
             load_lane(v, xr, lo, cnt, vb);
         }
-        // The lane's samples from zero state, in time order.
         double s1[SMAX], s2[SMAX];
-#pragma unroll
-        for (int i = 0; i < SMAX; ++i) s1[i] = s2[i] = 0.0;
-        if (__all(full)) {
-            if (!REV) {
-#pragma unroll
-                for (int k = 0; k < kGroup; ++k) v[k] = df2t_step<SMAX>(v[k], s1, s2, cf, S);
-            } else {
-#pragma unroll
-                for (int k = kGroup - 1; k >= 0; --k) v[k] = df2t_step<SMAX>(v[k], s1, s2, cf, S);
-            }
-        } else {
-            if (!REV) {
-#pragma unroll
-                for (int k = 0; k < kGroup; ++k)
-                    if (k < cnt) v[k] = df2t_step<SMAX>(v[k], s1, s2, cf, S);
-            } else {
-#pragma unroll
-                for (int k = kGroup - 1; k >= 0; --k)
-                    if (k < cnt) v[k] = df2t_step<SMAX>(v[k], s1, s2, cf, S);
-            }
-        }
+        filter_group<SMAX, REV>(v, cnt, __all(full), s1, s2, cf, S);
         double e[D];
 #pragma unroll
         for (int i = 0; i < SMAX; ++i) {
@@ -383,7 +536,7 @@ __global__ __launch_bounds__(kThreads) void sos_wave_kernel(
         const int last = (int)std::min<int64_t>(63, ngroups - 1 - st * 64);
 #pragma unroll
         for (int i = 0; i < D; ++i) zin[i] = __shfl(e[i], last, 64);
-        if (MODE == kRun) {
+        if (MODE != kState) {
             // y = y0 + C z; the chunk's very first lane starts from zero
             // (and keeps the reference's bits, signed zeros included).
             if (!(st == 0 && lane == 0 && c == 0)) {
@@ -418,6 +571,32 @@ __global__ __launch_bounds__(kThreads) void sos_wave_kernel(
 #pragma unroll
                 for (int k = 0; k < kGroup; ++k)
                     if (k < cnt) yr[lo + k] = v[k];
+            }
+            if constexpr (BACK) {
+                // The step's groups back to front: lane l's end state passes
+                // the l groups before it.
+                filter_group<SMAX, !REV>(v, cnt, __all(full), s1, s2, cf, S);
+                double b[D];
+#pragma unroll
+                for (int i = 0; i < SMAX; ++i) {
+                    b[2 * i] = s1[i];
+                    b[2 * i + 1] = s2[i];
+                }
+                reduce_down<D>(b, pwv, lane, ngroups - st * 64);
+#pragma unroll
+                for (int i = 0; i < D; ++i) {
+                    const double b0 = __shfl(b[i], 0, 64);
+                    back[i] = lane == st ? b0 : back[i];
+                }
+            }
+        }
+    }
+    if constexpr (BACK) {
+        if (c > 0) {  // chunk 0 is the other direction's last
+            reduce_down<D>(back, mats + mats_m(D), lane, nsteps);
+            if (lane == 0) {
+#pragma unroll
+                for (int i = 0; i < D; ++i) zs[((rows + row) * nC + nC - 1 - c) * D + i] = back[i];
             }
         }
     }
@@ -597,54 +776,84 @@ bool aligned_rows(const double *p, int64_t ld)
     return (reinterpret_cast<uintptr_t>(p) & 15) == 0 && (ld & 1) == 0;
 }
 
+// What sos_run decided about a call.
+struct SosPlan {
+    bool row_mode;    // one lane a row
+    bool collect;     // the RUN waves collect their start states
+    int64_t L, nC;    // chunk length, chunks a row
+    double *mats, *zs;
+};
+
 template <int SMAX, bool REV>
-int sos_launch_t(const double *x, int64_t ldx, double *y, int64_t ldy, int64_t rows, int64_t N,
-                 const double *sos, int S, bool row_mode, int64_t L, int64_t nC, double *mats,
-                 double *zs, int cu_count, hipStream_t s)
+int sos_direction(const double *x, int64_t ldx, double *y, int64_t ldy, int64_t rows, int64_t N,
+                  const double *sos, int S, const SosPlan &p, int cu_count, hipStream_t s)
 {
     const int vec = aligned_rows(x, ldx) && aligned_rows(y, ldy);
-    if (row_mode) {
+    if (p.row_mode) {
         // rows per wave: spread the rows over the CUs (one wave each) first
         const int rpw = (int)std::min<int64_t>(64, std::max<int64_t>(1, (rows + cu_count - 1) / cu_count));
         hipLaunchKernelGGL((sos_row_kernel<SMAX, REV>), dim3((unsigned)((rows + rpw - 1) / rpw)),
                            dim3(64), 0, s, x, ldx, y, ldy, rows, N, sos, S, vec, rpw);
         return check_launch("sos_row_kernel");
     }
-    hipLaunchKernelGGL((sos_setup_kernel<SMAX>), dim3(1), dim3(kThreads), 0, s, sos, S,
-                       nC > 1 ? L / kGroup : (int64_t)0, mats);
-    SCIR_TRY(check_launch("sos_setup_kernel"));
-    const int64_t waves = rows * nC;
+    const int64_t waves = rows * p.nC;
     const unsigned blocks = (unsigned)((waves + kThreads / 64 - 1) / (kThreads / 64));
-    if (nC > 1) {
+    if (p.nC > 1) {
         hipLaunchKernelGGL((sos_wave_kernel<SMAX, kState, REV>), dim3(blocks), dim3(kThreads), 0, s,
-                           x, ldx, y, ldy, rows, N, sos, S, L, nC, mats, zs, vec);
+                           x, ldx, y, ldy, rows, N, sos, S, p.L, p.nC, p.mats, p.zs, vec);
         SCIR_TRY(check_launch("sos_wave_kernel(state)"));
         hipLaunchKernelGGL((sos_scan_kernel<SMAX>), dim3((unsigned)((rows + 3) / 4)),
-                           dim3(kThreads), 0, s, zs, mats + mats_t(2 * SMAX), rows, nC, S);
+                           dim3(kThreads), 0, s, p.zs, p.mats + mats_t(2 * SMAX), rows, p.nC, S);
         SCIR_TRY(check_launch("sos_scan_kernel"));
     }
     hipLaunchKernelGGL((sos_wave_kernel<SMAX, kRun, REV>), dim3(blocks), dim3(kThreads), 0, s, x,
-                       ldx, y, ldy, rows, N, sos, S, L, nC, mats, nC > 1 ? zs : nullptr, vec);
+                       ldx, y, ldy, rows, N, sos, S, p.L, p.nC, p.mats,
+                       p.nC > 1 ? p.zs : nullptr, vec);
     return check_launch("sos_wave_kernel(run)");
 }
 
-template <bool REV>
-int sos_launch_rev(const double *x, int64_t ldx, double *y, int64_t ldy, int64_t rows, int64_t N,
-                   const double *sos, int S, bool row_mode, int64_t L, int64_t nC, double *mats,
-                   double *zs, int cu_count, hipStream_t s)
+template <int S>
+int sos_collect(const double *x, int64_t ldx, double *y, int64_t ldy, int64_t rows, int64_t N,
+                const double *sos, const SosPlan &p, bool zero_phase, hipStream_t s)
 {
-#define SCIR_SOS_CASE(n)                                                                     \
-    case n:                                                                                  \
-        return sos_launch_t<n, REV>(x, ldx, y, ldy, rows, N, sos, S, row_mode, L, nC, mats, \
-                                    zs, cu_count, s);
-    switch (S) {
-        SCIR_SOS_CASE(1) SCIR_SOS_CASE(2) SCIR_SOS_CASE(3) SCIR_SOS_CASE(4)
-        SCIR_SOS_CASE(5) SCIR_SOS_CASE(6) SCIR_SOS_CASE(7) SCIR_SOS_CASE(8)
-        default:
-            return sos_launch_t<kMaxSections, REV>(x, ldx, y, ldy, rows, N, sos, S, row_mode, L,
-                                                   nC, mats, zs, cu_count, s);
+    const int yv = aligned_rows(y, ldy), vec = aligned_rows(x, ldx) && yv;
+    const unsigned blocks = (unsigned)((rows * p.nC + kThreads / 64 - 1) / (kThreads / 64));
+    hipLaunchKernelGGL((sos_prepare_kernel<S>), dim3(1), dim3(64), 0, s, sos, p.L / kGroup, p.mats);
+    SCIR_TRY(check_launch("sos_prepare_kernel"));
+    hipLaunchKernelGGL((sos_wave_kernel<S, kState, false>), dim3(blocks), dim3(kThreads), 0, s, x,
+                       ldx, y, ldy, rows, N, sos, S, p.L, p.nC, p.mats, p.zs, vec);
+    SCIR_TRY(check_launch("sos_wave_kernel(state)"));
+    if (!zero_phase) {
+        hipLaunchKernelGGL((sos_wave_kernel<S, kCollect, false>), dim3(blocks), dim3(kThreads), 0,
+                           s, x, ldx, y, ldy, rows, N, sos, S, p.L, p.nC, p.mats, p.zs, vec);
+        return check_launch("sos_wave_kernel(collect)");
     }
-#undef SCIR_SOS_CASE
+    hipLaunchKernelGGL((sos_wave_kernel<S, kCollect, false, true>), dim3(blocks), dim3(kThreads),
+                       0, s, x, ldx, y, ldy, rows, N, sos, S, p.L, p.nC, p.mats, p.zs, vec);
+    SCIR_TRY(check_launch("sos_wave_kernel(collect, back)"));
+    hipLaunchKernelGGL((sos_wave_kernel<S, kCollect, true>), dim3(blocks), dim3(kThreads), 0, s, y,
+                       ldy, y, ldy, rows, N, sos, S, p.L, p.nC, p.mats, p.zs + rows * p.nC * 2 * S,
+                       yv);
+    return check_launch("sos_wave_kernel(collect, reverse)");
+}
+
+template <int SMAX>
+int sos_launch_t(const double *x, int64_t ldx, double *y, int64_t ldy, int64_t rows, int64_t N,
+                 const double *sos, int S, const SosPlan &p, bool zero_phase, int cu_count,
+                 hipStream_t s)
+{
+    if constexpr (SMAX <= kCollectMaxS)
+        if (p.collect)
+            return sos_collect<SMAX>(x, ldx, y, ldy, rows, N, sos, p, zero_phase, s);
+    if (!p.row_mode) {
+        hipLaunchKernelGGL((sos_setup_kernel<SMAX>), dim3(1), dim3(kThreads), 0, s, sos, S,
+                           p.nC > 1 ? p.L / kGroup : (int64_t)0, p.mats);
+        SCIR_TRY(check_launch("sos_setup_kernel"));
+    }
+    SCIR_TRY((sos_direction<SMAX, false>(x, ldx, y, ldy, rows, N, sos, S, p, cu_count, s)));
+    return zero_phase
+               ? sos_direction<SMAX, true>(y, ldy, y, ldy, rows, N, sos, S, p, cu_count, s)
+               : SCIR_HIP_OK;
 }
 
 }  // namespace
@@ -671,9 +880,18 @@ void sos_plan(int64_t rows, int64_t N, int cu_count, bool reference_order, bool 
     *nC = (N + l - 1) / l;
 }
 
-// Runs one direction (caller holds st->mu).
+// Whether a plan's RUN waves collect their start states: up to kMaxChunks
+// chunks a row, four sections (a lane per matrix element in
+// sos_prepare_kernel), and chunks of up to kMaxSteps steps when the outputs
+// also run back to front (a lane keeps each step's state).
+bool sos_collects(int64_t L, int64_t nC, int S)
+{
+    return S <= kCollectMaxS && nC > 1 && nC <= kMaxChunks && L <= kMaxSteps * kStep;
+}
+
+// Forward, and for zero_phase back over the result (caller holds st->mu).
 int sos_run(const double *x, int64_t ldx, double *y, int64_t ldy, int64_t rows, int64_t N,
-            const double *sos, int S, bool reference_order, bool rev, hipStream_t s,
+            const double *sos, int S, bool reference_order, bool zero_phase, hipStream_t s,
             DeviceState *st)
 {
     if (S == 0) {  // no sections: the cascade passes its input through
@@ -682,27 +900,40 @@ int sos_run(const double *x, int64_t ldx, double *y, int64_t ldy, int64_t rows, 
                                           N * sizeof(double), rows, hipMemcpyDeviceToDevice, s));
         return SCIR_HIP_OK;
     }
-    bool row_mode = false;
-    int64_t L = 0, nC = 0;
-    sos_plan(rows, N, st->cu_count, reference_order, &row_mode, &L, &nC);
-    if ((row_mode ? rows : rows * nC / (kThreads / 64)) + 2 > 0x7fffffffLL)
+    SosPlan p{};
+    sos_plan(rows, N, st->cu_count, reference_order, &p.row_mode, &p.L, &p.nC);
+    if ((p.row_mode ? rows : rows * p.nC / (kThreads / 64)) + 2 > 0x7fffffffLL)
         return fail(SCIR_HIP_ERR_INVALID_ARGUMENT, "too many rows");
-    double *mats = nullptr, *zs = nullptr;
-    if (!row_mode) {
+    if (!p.row_mode) {
         StreamScratch &sc = scratch_for(st, s);
         const int d = 2 * S;
         const int Dk = 2 * (S <= 8 ? S : kMaxSections);  // the kernels' padded dimension
-        const int64_t mdoubles = (mats_size(Dk, d) + 31) / 32 * 32;
-        const int64_t zdoubles = nC > 1 ? rows * nC * d : 0;
+        auto up32 = [](int64_t v) { return (v + 31) / 32 * 32; };
+        int64_t mdoubles = up32(collect_mats_size(d));
+        int64_t zdoubles = 2 * rows * p.nC * d;  // both directions
+        // A capture cannot allocate, and the scan needs less scratch.
+        p.collect = sos_collects(p.L, p.nC, S) &&
+                    (!stream_capturing(s) ||
+                     (mdoubles + zdoubles) * sizeof(double) <= sc.sos_states.bytes);
+        if (!p.collect) {
+            mdoubles = up32(mats_size(Dk, d));
+            zdoubles = p.nC > 1 ? rows * p.nC * d : 0;
+        }
         SCIR_TRY(ensure_scratch(st, sc.sos_states, (size_t)(mdoubles + zdoubles) * sizeof(double), s));
-        mats = static_cast<double *>(sc.sos_states.ptr);
-        zs = mats + mdoubles;
+        p.mats = static_cast<double *>(sc.sos_states.ptr);
+        p.zs = p.mats + mdoubles;
     }
-    if (rev)
-        return sos_launch_rev<true>(x, ldx, y, ldy, rows, N, sos, S, row_mode, L, nC, mats, zs,
-                                    st->cu_count, s);
-    return sos_launch_rev<false>(x, ldx, y, ldy, rows, N, sos, S, row_mode, L, nC, mats, zs,
-                                 st->cu_count, s);
+    switch (S) {
+#define SCIR_SOS_CASE(n)                                                                  \
+    case n:                                                                               \
+        return sos_launch_t<n>(x, ldx, y, ldy, rows, N, sos, S, p, zero_phase, st->cu_count, s);
+        SCIR_SOS_CASE(1) SCIR_SOS_CASE(2) SCIR_SOS_CASE(3) SCIR_SOS_CASE(4)
+        SCIR_SOS_CASE(5) SCIR_SOS_CASE(6) SCIR_SOS_CASE(7) SCIR_SOS_CASE(8)
+#undef SCIR_SOS_CASE
+    default:
+        return sos_launch_t<kMaxSections>(x, ldx, y, ldy, rows, N, sos, S, p, zero_phase,
+                                          st->cu_count, s);
+    }
 }
 
 int sos_args(const double *x, int64_t ldx, int64_t rows, int64_t N, const double *sos, int32_t S,
@@ -739,9 +970,7 @@ int sos_dev(const double *x, int64_t ldx, int64_t rows, int64_t N, const double 
     std::lock_guard<std::mutex> lk(st->mu);
     const bool ref = (flags & SCIR_HIP_SOS_REFERENCE_ORDER) != 0;
     hipStream_t s = as_stream(stream);
-    SCIR_TRY(sos_run(x, ldx, y, ldy, rows, N, sos, S, ref, false, s, st));
-    if (zero_phase) SCIR_TRY(sos_run(y, ldy, y, ldy, rows, N, sos, S, ref, true, s, st));
-    return SCIR_HIP_OK;
+    return sos_run(x, ldx, y, ldy, rows, N, sos, S, ref, zero_phase, s, st);
 }
 
 int sos_host(const double *x, int64_t ldx, int64_t rows, int64_t N, const double *sos, int32_t S,
@@ -767,8 +996,7 @@ int sos_host(const double *x, int64_t ldx, int64_t rows, int64_t N, const double
                                     hipMemcpyHostToDevice, s));
     // In place on the device copy: each chunk is read before it is written.
     const bool ref = (flags & SCIR_HIP_SOS_REFERENCE_ORDER) != 0;
-    SCIR_TRY(sos_run(dx, N, dx, N, rows, N, dsos, S, ref, false, s, st));
-    if (zero_phase) SCIR_TRY(sos_run(dx, N, dx, N, rows, N, dsos, S, ref, true, s, st));
+    SCIR_TRY(sos_run(dx, N, dx, N, rows, N, dsos, S, ref, zero_phase, s, st));
     SCIR_HIP_TRY(hipMemcpy2DAsync(y, ldy * sizeof(double), dx, row_bytes, row_bytes, rows,
                                   hipMemcpyDeviceToHost, s));
     SCIR_HIP_TRY(hipStreamSynchronize(s));

@@ -142,3 +142,73 @@ def test_full_size_rows():
         _check(y[r].cpu().numpy()[None, :], ref[None, :], True)
     del x, y
     torch.cuda.empty_cache()
+
+
+# Few rows run in chunks of 1024 or 2048 samples that a wave holds: one chunk
+# and its edges, 64, 65 and 128 of each (a lane collects two states), the first
+# row length beyond them, rows enough to take the longer chunks, odd pitches.
+@pytest.mark.parametrize("S", [1, 2, 3, 4])
+@pytest.mark.parametrize("rows,n", [(1, 1025), (3, 2048), (2, 2049), (1, 65536), (2, 65537),
+                                    (1, 131072), (1, 131073), (2, 262144), (1, 262145),
+                                    (40, 130001), (700, 6001), (4095, 1100)])
+def test_register_chunks(S, rows, n):
+    print(f"sosfilt register chunks S={S} rows={rows} n={n}", flush=True)
+    x = np.random.default_rng(S + n).standard_normal((rows, n))
+    sos = _sos(S, S + n)
+    keep = sorted({0, rows // 2, rows - 1})
+    want, zero = orc.sosfilt_f64(sos, x[keep]), orc.filtfilt_f64(sos, x[keep])
+    sos_t = torch.tensor(sos, device="cuda")
+    for pitch in (n, n + 1):
+        buf = torch.zeros((rows, pitch), dtype=torch.float64, device="cuda")
+        xt = buf[:, :n]
+        xt.copy_(torch.tensor(x))
+        out = torch.full((rows, pitch), np.nan, dtype=torch.float64, device="cuda")[:, :n]
+        device.sosfilt(xt, sos_t, out=out)
+        _check(out.cpu().numpy()[keep], want, True, sos, x[keep])
+        device.sosfilt(xt, sos_t, zero_phase=True, out=out)
+        _check(out.cpu().numpy()[keep], zero, False, sos, x[keep], zero_phase=True)
+        device.sosfilt(xt, sos_t, zero_phase=True, out=xt)  # in place
+        _check(xt.cpu().numpy()[keep], zero, False, sos, x[keep], zero_phase=True)
+
+
+def test_register_chunks_unstable_and_nonfinite():
+    """A growing filter whose transition powers overflow (2000 of them would,
+    the row is shorter), and NaNs: finite exactly before the first."""
+    r = np.random.default_rng(3)
+    sos = np.array([[1.0, 0.2, 0.1, 1.0, -2 * 1.05 * np.cos(0.3), 1.05 ** 2]])
+    x = r.standard_normal((3, 5000))
+    print("sosfilt register chunks unstable", flush=True)
+    y, ref = signal.sosfilt_batched(sos, x, Device.Hip), orc.sosfilt_f64(sos, x)
+    assert np.all(np.isfinite(ref))
+    # Compared where the reference loop is: the output grows 1e100 times over.
+    run = np.maximum.accumulate(np.abs(ref), axis=1)
+    assert np.max(np.abs(y - ref) / run) <= 1e-9
+    x[1, 3000] = np.nan
+    y = signal.sosfilt_batched(sos, x, Device.Hip)
+    assert np.all(np.isfinite(y[1, :3000])) and np.all(np.isnan(y[1, 3000:]))
+    assert np.all(np.isfinite(y[[0, 2]]))
+
+
+def test_register_chunks_captured_with_small_scratch():
+    """A capture whose stream's scratch holds the general path's states but
+    not both directions': it is taken, and replays to the oracle's results."""
+    n, sos = 131072, _sos(1, 5)
+    g = torch.Generator(device="cuda").manual_seed(4)
+    x = torch.randn((1, n), device="cuda", dtype=torch.float64, generator=g)
+    sos_t, y = torch.tensor(sos, device="cuda"), torch.empty_like(x)
+    print("sosfilt capture with small scratch", flush=True)
+    st = torch.cuda.Stream()
+    st.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(st):
+        device.sosfilt(x[:, :1025].contiguous(), sos_t, zero_phase=True)
+        st.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=st):
+            device.sosfilt(x, sos_t, zero_phase=True, out=y)
+    for _ in range(3):
+        x.copy_(torch.randn((1, n), device="cuda", dtype=torch.float64, generator=g))
+        y.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        xh = x.cpu().numpy()
+        _check(y.cpu().numpy(), orc.filtfilt_f64(sos, xh), False, sos, xh, zero_phase=True)
