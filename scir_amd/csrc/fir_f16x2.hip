@@ -90,6 +90,10 @@ __device__ __forceinline__ float pow2(int e)  // |e| <= 126
 {
     return __builtin_bit_cast(float, (unsigned int)(e + 127) << 23);
 }
+__device__ __forceinline__ SplitScale split_scale(int s)  // |s| <= 100
+{
+    return {pow2(s), pow2(-s), pow2(s + 11)};
+}
 __device__ __forceinline__ int wave_umax(unsigned int v)
 {
     return wave_reduce((int)v, [](int a, int b) { return (int)max((unsigned)a, (unsigned)b); });
@@ -104,6 +108,13 @@ __device__ __forceinline__ float uniform(float v)
     return __builtin_bit_cast(float, uniform(__builtin_bit_cast(int, v)));
 }
 
+// min(a, |b|, |c|), NaN if any is: one v_minimum3_f32.
+__device__ __forceinline__ float minimum3(float a, float b, float c)
+{
+    return __builtin_elementwise_minimum(
+        __builtin_elementwise_minimum(__builtin_fabsf(b), __builtin_fabsf(c)), a);
+}
+
 // Scale exponent that puts a largest magnitude (bits mx) in [2^13, 2^14).
 __device__ __forceinline__ int scale_exponent(unsigned int mx)
 {
@@ -113,16 +124,19 @@ __device__ __forceinline__ int scale_exponent(unsigned int mx)
 // Splits the 8 samples of unit u into the two split arrays.
 template <int TW, bool REV>
 __device__ __forceinline__ void store_unit2(unsigned char *lds, int stride, int u,
-                                            const f32x4 (&r)[2], float scale)
+                                            const f32x4 (&r)[2], const SplitScale &scale)
 {
     unsigned int w[2][4];
 #pragma unroll
-    for (int p = 0; p < 4; ++p) {
-        unsigned int h, l;
-        split2_pair(r[p >> 1][2 * (p & 1)], r[p >> 1][2 * (p & 1) + 1], scale, h, l);
-        const int q = REV ? 3 - p : p;  // as in store_unit
-        w[0][q] = REV ? __builtin_amdgcn_alignbit(h, h, 16) : h;
-        w[1][q] = REV ? __builtin_amdgcn_alignbit(l, l, 16) : l;
+    for (int p = 0; p < 4; p += 2) {
+        unsigned int h[2], l[2];
+        split2_quad(r[p >> 1], scale, h, l);
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            const int q = REV ? 3 - p - e : p + e;  // as in store_unit
+            w[0][q] = REV ? __builtin_amdgcn_alignbit(h[e], h[e], 16) : h[e];
+            w[1][q] = REV ? __builtin_amdgcn_alignbit(l[e], l[e], 16) : l[e];
+        }
     }
 #pragma unroll
     for (int s = 0; s < 2; ++s)
@@ -155,7 +169,8 @@ struct SplitGroup {
     __device__ __forceinline__ void build_two()
     {
         int unused = 0;
-        build_tap_table<2, TW>(lds, lay.tab_offset, lay.copy2, b, K, m_hi, unused, pow2(sb));
+        build_tap_table<2, TW>(lds, lay.tab_offset, lay.copy2, b, K, m_hi, unused,
+                               split_scale(sb));
         table = kTwo;
     }
 
@@ -165,21 +180,20 @@ struct SplitGroup {
     __device__ __forceinline__ void measure(const f32x4 (&raw)[PF][2], int64_t N, int64_t xb,
                                             int tid)
     {
-        unsigned int mx = 0, mn = 0x7fffffffu;
+        float largest = 0.0f, least = __builtin_inff();  // NaN once there is one
+        unsigned int mn;
         const int n = units();
 #pragma unroll
         for (int j = 0; j < PF; ++j) {
             if (tid + j * kThreads >= n) break;
 #pragma unroll
             for (int c = 0; c < 8; c += 2) {
-                const unsigned int a0 = abs_bits(raw[j][c >> 2][c & 3]);
-                const unsigned int a1 = abs_bits(raw[j][c >> 2][(c & 3) + 1]);
-                mx = max(mx, max(a0, a1));
-                mn = min(mn, min(a0, a1));
+                largest = maximum3(largest, raw[j][c >> 2][c & 3], raw[j][c >> 2][(c & 3) + 1]);
+                least = minimum3(least, raw[j][c >> 2][c & 3], raw[j][c >> 2][(c & 3) + 1]);
             }
         }
-        const int wmx = wave_umax(mx);
-        int wmn = wave_umin(mn), we;
+        const int wmx = wave_umax(abs_bits(largest));
+        int wmn = wave_umin(abs_bits(least)), we;
         if (wmn != 0) {
             we = __builtin_amdgcn_frexp_expf(__builtin_bit_cast(float, wmn));
         } else {
@@ -370,17 +384,20 @@ struct SplitGroup {
                                             int tid, Next next)
     {
         const int wave = tid >> 6, lane = tid & 63;
-        if (fit(P0 < (m_hi + 1) / 2)) {
+        const bool two = fit(P0 < (m_hi + 1) / 2);
+        if (two) {
             if (table != kTwo) build_two();
-            const float scale = pow2(sx);
+            const SplitScale scale = split_scale(sx);
             const int n = units();
 #pragma unroll
             for (int j = 0; j < PF; ++j) {
                 const int u = tid + j * kThreads;
                 if (u < n) store_unit2<TW, REV>(lds, lay.stride2, u, raw[j], scale);
             }
-            __syncthreads();
-            next();
+        }
+        __syncthreads();
+        next();
+        if (two) {
             // A wave past the row end has no output (see fir_mfma_kernel).
             if (32 * (P0 + (int64_t)uniform(wave) * 32 * TW) < N) {
                 const int i = lane & 31, g = lane >> 5;
@@ -396,7 +413,6 @@ struct SplitGroup {
 #pragma unroll 1
         for (int h = 0; h < TW; ++h)
             if (32 * (P0 + 128 * h) < N) half_three(xrow, yrow, N, P0 + 128 * h, wave, lane);
-        next();
     }
 };
 
@@ -411,35 +427,46 @@ __global__ __launch_bounds__(kThreads, 2) void fir_f16x2_kernel(
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
     using Group = SplitGroup<TW, REV>;
     const int64_t seg_first = xcd_remap(blockIdx.x, nwg) * segs_per_wg;
-    const int64_t seg_end = min(nsegs, seg_first + segs_per_wg);
+    const int count = (int)min((int64_t)segs_per_wg, nsegs - seg_first);
+    // Row and segment of the row, stepped: a 64-bit division is some 150
+    // scalar instructions, and one stood before every contraction.
+    const int64_t first_row = seg_first / segs_per_row;
+    int seg = (int)(seg_first - first_row * segs_per_row);
+    const float *xrow = x + (row0 + first_row) * ldx;
+    float *yrow = y + (row0 + first_row) * ldy;
     f32x4 raw[Group::PF][2];
-    auto prefetch = [&](int64_t sg, int tid) {
-        const float *xrow = x + (row0 + sg / segs_per_row) * ldx;
-        const int64_t xb = 32 * (sg % segs_per_row) * Group::SEG_BLOCKS - 16 * (int64_t)m_hi;
+    auto prefetch = [&](const float *xr, int sg, int tid) {
+        const int64_t xb = 32 * (int64_t)sg * Group::SEG_BLOCKS - 16 * (int64_t)m_hi;
 #pragma unroll
         for (int j = 0; j < Group::PF; ++j)
-            load_unit<REV>(xrow, N, xb, tid + j * kThreads, Group::SEG_BLOCKS * 4 + 2 * m_hi,
+            load_unit<REV>(xr, N, xb, tid + j * kThreads, Group::SEG_BLOCKS * 4 + 2 * m_hi,
                            raw[j]);
     };
-    prefetch(seg_first, (int)threadIdx.x);
+    prefetch(xrow, seg, (int)threadIdx.x);
     Group group;
     group.lds = lds;
     group.lay = lay;
-    group.begin(b, K, false, raw, N, (seg_first % segs_per_row) * Group::SEG_BLOCKS);
-    for (int64_t sg = seg_first; sg < seg_end; ++sg) {
+    group.begin(b, K, false, raw, N, (int64_t)seg * Group::SEG_BLOCKS);
+    for (int done = 0; done < count; ++done) {
         // Lane-dependent values are recomputed in every iteration (see
         // fir_mfma_kernel).
         int tid = (int)threadIdx.x;
         asm volatile("" : "+v"(tid));
-        const int64_t row = row0 + sg / segs_per_row;
-        const int64_t P0 = (sg % segs_per_row) * Group::SEG_BLOCKS;
-        if (sg != seg_first) {
+        const int64_t P0 = (int64_t)seg * Group::SEG_BLOCKS;
+        if (done) {
             group.measure(raw, N, 32 * P0 - 16 * (int64_t)m_hi, tid);
             __syncthreads();  // the previous segment's MFMAs are done
         }
-        group.segment(raw, x + row * ldx, y + row * ldy, N, P0, tid, [&] {
-                          if (sg + 1 < seg_end) prefetch(sg + 1, tid);
-                      });
+        const bool last = seg + 1 == segs_per_row;
+        const int next_seg = last ? 0 : seg + 1;
+        group.segment(raw, xrow, yrow, N, P0, tid, [&] {
+            if (done + 1 < count) prefetch(last ? xrow + ldx : xrow, next_seg, tid);
+        });
+        seg = next_seg;
+        if (last) {
+            xrow += ldx;
+            yrow += ldy;
+        }
     }
 }
 

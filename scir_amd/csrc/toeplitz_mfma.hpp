@@ -149,20 +149,39 @@ __device__ __forceinline__ void split3_pair(float v0, float v1, unsigned int &h,
 }
 
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
-constexpr float kLoScale = 2048.0f;          // 2^11: the low term's scale
-constexpr float kLoUnscale = 1.0f / 2048.0f;
+constexpr float kLoUnscale = 1.0f / 2048.0f;  // 2^-11: the low term's scale is 2^11
 
-// The two fp16 terms, as packed words, of v0 * scale and v1 * scale (scale a
-// power of two).
-__device__ __forceinline__ void split2_pair(float v0, float v1, float scale, unsigned int &h,
-                                            unsigned int &l)
+// The powers of two of an F16x2 split, of samples or taps.
+struct SplitScale {
+    float to;       // 2^s
+    float from;     // 2^-s
+    float to_lo;    // 2^(s + 11)
+};
+
+// The two fp16 terms, as packed words, of four values: three mixed-precision
+// multiply-adds a value (hi = rn(2^s v); v - 2^-s hi, exact; lo), where the
+// compiler's choice takes four and a half.  Each write of half a register is
+// one instruction away from the next use of that register, as the hardware
+// requires.
+__device__ __forceinline__ void split2_quad(const f32x4 &v, const SplitScale &c,
+                                            unsigned int (&h)[2], unsigned int (&l)[2])
 {
-    const f16x2 hi = __builtin_convertvector(f32x2{v0 * scale, v1 * scale}, f16x2);
-    // 2^11 (v scale - hi), exactly: a mixed-precision multiply-add.
-    const f32x2 r = {__builtin_fmaf((float)hi.x, -kLoScale, v0 * (scale * kLoScale)),
-                     __builtin_fmaf((float)hi.y, -kLoScale, v1 * (scale * kLoScale))};
-    h = __builtin_bit_cast(unsigned int, hi);
-    l = __builtin_bit_cast(unsigned int, __builtin_convertvector(r, f16x2));
+    float r1, r3;
+    asm("v_fma_mixlo_f16 %0, %6, %10, 0\n\t"
+        "v_fma_mixlo_f16 %1, %8, %10, 0\n\t"
+        "v_fma_mixhi_f16 %0, %7, %10, 0\n\t"
+        "v_fma_mixhi_f16 %1, %9, %10, 0\n\t"
+        "v_fma_mix_f32 %2, %0, -%11, %6 op_sel_hi:[1,0,0]\n\t"
+        "v_fma_mix_f32 %4, %0, -%11, %7 op_sel:[1,0,0] op_sel_hi:[1,0,0]\n\t"
+        "v_fma_mix_f32 %3, %1, -%11, %8 op_sel_hi:[1,0,0]\n\t"
+        "v_fma_mix_f32 %5, %1, -%11, %9 op_sel:[1,0,0] op_sel_hi:[1,0,0]\n\t"
+        "v_fma_mixlo_f16 %2, %2, %12, 0\n\t"
+        "v_fma_mixlo_f16 %3, %3, %12, 0\n\t"
+        "v_fma_mixhi_f16 %2, %4, %12, 0\n\t"
+        "v_fma_mixhi_f16 %3, %5, %12, 0\n\t"
+        "s_nop 0"
+        : "=&v"(h[0]), "=&v"(h[1]), "=&v"(l[0]), "=&v"(l[1]), "=&v"(r1), "=&v"(r3)
+        : "v"(v.x), "v"(v.y), "v"(v.z), "v"(v.w), "s"(c.to), "s"(c.from), "s"(c.to_lo));
 }
 
 __device__ __forceinline__ unsigned int pack2(unsigned short lo, unsigned short hi)
@@ -221,6 +240,13 @@ __device__ __forceinline__ bool segment_is_tiny(const int *mins)
     const int ex = min(min(mins[0], mins[1]), min(mins[2], mins[3]));
     const int eb = min(min(mins[4], mins[5]), min(mins[6], mins[7]));
     return tiny_magnitudes(ex, eb);
+}
+
+// max(a, |b|, |c|), NaN if any is: one v_maximum3_f32.
+__device__ __forceinline__ float maximum3(float a, float b, float c)
+{
+    return __builtin_elementwise_maximum(
+        __builtin_elementwise_maximum(__builtin_fabsf(b), __builtin_fabsf(c)), a);
 }
 
 template <int S>
@@ -424,8 +450,16 @@ struct Contraction {
     __device__ __forceinline__ void run()
     {
         const int half = CH == 2 ? msteps / 2 : msteps;  // msteps >= 2
+        // Two passes: of the two waves on a SIMD, the one that is further on
+        // goes first, up to its next contraction.  Equal shares keep the two
+        // in step, and staging and stores of both then meet (K = 512: 1780 ->
+        // 1733 us, 1023: 374 -> 355).
+        if constexpr (CH == 2) __builtin_amdgcn_s_setprio(0);
         pass<0>(half);
-        if constexpr (CH == 2) pass<1>(msteps - half);
+        if constexpr (CH == 2) {
+            __builtin_amdgcn_s_setprio(1);
+            pass<1>(msteps - half);
+        }
     }
 };
 
@@ -516,7 +550,8 @@ __device__ __forceinline__ void store_unit(unsigned char *lds, int split_stride,
 template <int S, int TW>
 __device__ __forceinline__ void build_tap_table(unsigned char *lds, int tab_offset,
                                                 int copy_bytes, const float *__restrict__ b,
-                                                int K, int m_hi, int &min_b, float scale = 1.0f)
+                                                int K, int m_hi, int &min_b,
+                                                const SplitScale &scale = {})
 {
     const int C = 16 * (m_hi + 2 * TW + 1) + 32, L = C + 32 * TW + 32;
     constexpr int R = 4;
@@ -537,10 +572,10 @@ __device__ __forceinline__ void build_tap_table(unsigned char *lds, int tab_offs
             if (S == 3) {
                 split3(v[r], t[0], t[1], t[2]);
             } else if (S == 2) {
-                unsigned int h, l;
-                split2_pair(v[r], 0.0f, scale, h, l);
-                t[0] = (unsigned short)h;
-                t[1] = (unsigned short)l;
+                const _Float16 hi = (_Float16)(v[r] * scale.to);
+                t[0] = f16_bits(hi);
+                t[1] = f16_bits((_Float16)(__builtin_fmaf((float)hi, -scale.from, v[r]) *
+                                           scale.to_lo));
             } else {
                 t[0] = f16_bits((_Float16)v[r]);
             }
@@ -648,12 +683,12 @@ __device__ __forceinline__ void store_segment(const Contraction<S, TW> &ct,
         return S == 2 ? __builtin_ldexpf(v, out_exp) : v;
     };
     // Every output of the wave inside the row (a wave-uniform test): the
-    // stores go out unconditionally, one class test per output sets a flag,
-    // and only a flagged (or tiny) segment runs the recomputation pass over
+    // stores go out unconditionally, half an instruction per output notes a
+    // non-finite one, and only such (or tiny) segment runs the recomputation pass over
     // the stored values (rolled loops: indexing the accumulators there would
     // put them in scratch).
     if (32 * (P0 + (int64_t)(wave + 1) * 32 * TW) <= N) {
-        bool bad = false;
+        float largest = 0.0f;  // NaN once there is one
 #pragma unroll
         for (int t = 0; t < TW; ++t) {
             const int64_t n0 = 32 * (P0 + wave * 32 * TW + t + TW * i) + 4 * g;
@@ -662,8 +697,7 @@ __device__ __forceinline__ void store_segment(const Contraction<S, TW> &ct,
                 f32x4 v;
 #pragma unroll
                 for (int j = 0; j < 4; ++j) v[j] = output(t, 4 * q + j);
-                bad |= !__builtin_isfinite(v.x) | !__builtin_isfinite(v.y) |
-                       !__builtin_isfinite(v.z) | !__builtin_isfinite(v.w);
+                largest = maximum3(maximum3(largest, v.x, v.y), v.z, v.w);
                 const int64_t n = n0 + 8 * q;
                 if (!REV)
                     *reinterpret_cast<f32x4u *>(yrow + n) = v;
@@ -671,7 +705,7 @@ __device__ __forceinline__ void store_segment(const Contraction<S, TW> &ct,
                     *reinterpret_cast<f32x4u *>(yrow + (N - 4 - n)) = f32x4{v.w, v.z, v.y, v.x};
             }
         }
-        if (tiny || bad) {
+        if (tiny || !__builtin_isfinite(largest)) {
 #pragma unroll 1
             for (int t = 0; t < TW; ++t) {
                 const int64_t n0 = 32 * (P0 + wave * 32 * TW + t + TW * i) + 4 * g;
