@@ -116,10 +116,12 @@ int fir_mfma_dev(const float *x, int64_t ldx, const float *b, int K, int64_t B, 
                  float *y, int64_t ldy, int precision, bool rev, hipStream_t stream,
                  DeviceState *st);
 // F32 by two fp16 terms (fir_f16x2.hip): whether it takes K taps (its LDS
-// leaves room for two workgroups a CU), and the filter itself.
+// leaves room for two workgroups a CU), and the filter itself, as_ragged in the
+// ragged kernel's segments (the samples' scale is a segment's: the same bits).
 bool fir_f16x2_takes(int K);
 int fir_f16x2_dev(const float *x, int64_t ldx, const float *b, int K, int64_t B, int64_t N,
-                  float *y, int64_t ldy, bool rev, hipStream_t stream, DeviceState *st);
+                  float *y, int64_t ldy, bool rev, bool as_ragged, hipStream_t stream,
+                  DeviceState *st);
 // Partial sums (floats) the allocation-free dL/db entry point holds: 4 MiB.
 constexpr size_t kVjpNoAllocPartials = (size_t)1 << 20;
 // Device address of that entry point's scratch array on the current device.

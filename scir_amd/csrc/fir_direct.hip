@@ -592,13 +592,23 @@ int fir_direct_dev(const float *x, int64_t ldx, const float *b, int K, int64_t B
         // Default strips, measured on [4096, 65536]: 4 tiles at K = 1 (319 us
         // against 352 with 8), 8 at K = 17-33, 16 at K = 48, 32 from K = 64;
         // on [2048, 262144] 64 above K = 257 (K = 512: 5559 us, 5640 with 32).
-        const int strip = tc.direct_mfma_strip > 0 ? tc.direct_mfma_strip
-                          : K <= 8                 ? 4
-                          : K <= 40                ? 8
-                          : K <= 56                ? 16
-                          : K <= 257               ? 32
-                                                   : 64;
-        return launch_direct_mfma_k(x, ldx, b, K, B, N, y, ldy, strip, rev, stream);
+        // Smaller batches take shorter ones: a wave's tiles follow each other
+        // (a chain of 4 (K + 15) / 16 dependent products each), so 2048 waves
+        // come before tiles per wave, and 4096 before more than two (K = 31
+        // and 129: [1, 262144] 5.3 -> 3.0 us and 35 -> 4.3, [64, 16384] 5.8 ->
+        // 4.1 and 35 -> 6.7; [64, 65536] 8.1 and 36 -> 16), evened out over
+        // the row.
+        int64_t strip = tc.direct_mfma_strip;
+        if (strip <= 0) {
+            const int64_t row_tiles = (N + kMfmaTile - 1) / kMfmaTile, tiles = B * row_tiles;
+            strip = K <= 8 ? 4 : K <= 40 ? 8 : K <= 56 ? 16 : K <= 257 ? 32 : 64;
+            const int64_t fill =
+                std::max(std::min<int64_t>((tiles + 1024) / 2048, 2), (tiles + 2048) / 4096);
+            strip = std::max<int64_t>(1, std::min({strip, fill, row_tiles}));
+            const int64_t spr = (row_tiles + strip - 1) / strip;
+            strip = (row_tiles + spr - 1) / spr;
+        }
+        return launch_direct_mfma_k(x, ldx, b, K, B, N, y, ldy, (int)strip, rev, stream);
     }
     // LDS-DMA loader: forward rows, 16-byte aligned, N % 4 == 0, N < 2^29.
     if (tc.direct_loader >= 2 && K <= kPipeMaxK && !rev && N % 4 == 0 &&
@@ -635,21 +645,23 @@ namespace {
 //   * Above 513 taps, the end of the FP32 matrix-core kernel, always: the VALU
 //     form it replaces is slower at every size ([1, 5000], K = 1023: 21.3 ->
 //     17.0 us; [1024, 65536], K = 1023: 1810 -> 378 us).
-//   * Up to 513 the two cost about staged * (27 + ng) against 5 * outputs * ng
-//     (staged: whole segments; ng: groups of 16 taps), which crosses at K = 97
-//     on long rows ([4096, 65536]: 445 / 509 us at K = 65, 698 / 540 at 129,
-//     1274 / 655 at 255), later where rows fill their segments badly
-//     ([4000, 1000], K = 255: 28 / 43 us), and below 2^25 outputs * ng the
-//     FP32 kernel's shorter start wins ([64, 16384], K = 255: 10.3 / 10.8 us;
-//     at K = 512, 22.1 / 12.7).
+//   * Up to 513 the two cost about staged * (27 + ng) against c * outputs * ng
+//     (staged: whole segments; ng: groups of 16 taps), c = 5 up to K = 257 and
+//     8 above, where the FP32 kernel needs a second tile of history.  They
+//     cross at K = 97 on long rows ([4096, 65536]: 445 / 480 us at K = 65, 698
+//     / 515 at 129, 1274 / 620 at 255; [64, 65536]: 10.6 / 13.1, 16.4 / 14.2,
+//     27 / 16), later where rows fill their segments badly ([4000, 1000]: 29 /
+//     41 us at K = 255, 48 / 45 at 400, 58 / 49 at 512), and below 2^24 outputs
+//     * ng the FP32 kernel's shorter start wins ([64, 16384]: 8.9 / 8.4 us at
+//     K = 200, 14.2 / 9.6 at 400; [1, 262144], K = 400: 8.1 / 8.5).
 bool takes_f16x2(const TuneChoice &tc, int K, int64_t B, int64_t N)
 {
     if (tc.direct_loader != 3 || tc.direct_mfma_strip_forced || !fir_f16x2_takes(K)) return false;
     if (K > kMfmaF32MaxK) return true;
-    const int64_t ng = (K + 14) / 16 + 1;
+    const int64_t ng = (K + 14) / 16 + 1, c = K <= 257 ? 5 : 8;
     const int64_t seg = N <= 4096 ? 4096 : 8192;
     const int64_t staged = B * ((N + seg - 1) / seg) * seg;
-    return B * N * ng >= (int64_t)1 << 25 && staged * (27 + ng) < 5 * B * N * ng;
+    return B * N * ng >= (int64_t)1 << 24 && staged * (27 + ng) < c * B * N * ng;
 }
 
 // AUTO chooses between BF16x3 and F32 from its cut-over up.  By two fp16 terms
@@ -684,7 +696,7 @@ int fir_f32_dev(const float *x, int64_t ldx, const float *b, int K, int64_t B, i
 {
     const TuneChoice tc = tune_lookup(K, N);
     if (takes_f16x2(tc, K, B, N))
-        return fir_f16x2_dev(x, ldx, b, K, B, N, y, ldy, rev, stream, st);
+        return fir_f16x2_dev(x, ldx, b, K, B, N, y, ldy, rev, false, stream, st);
     if (takes_bf16x3(tc, K, B, N))
         return fir_mfma_dev(x, ldx, b, K, B, N, y, ldy, SCIR_HIP_PREC_BF16X3, rev, stream, st);
     return fir_direct_dev(x, ldx, b, K, B, N, y, ldy, false, rev, stream, st);

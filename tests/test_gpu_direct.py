@@ -266,3 +266,28 @@ def test_f32_mfma_boundaries_both_directions(hip, oracle, strip, K):
             assert np.all(np.abs(dx - dx64) <= bound), f"dL/dx N={N}"
     finally:
         hip.check(L.scir_hip_tune_set(b"direct.mfma_strip", -1))
+
+
+# Default strips by size: of one tile, two (from 3072 tiles of the batch), more
+# (from 6144), evened out over a row that they do not divide, short last tiles.
+@pytest.mark.parametrize("K", [1, 33, 129, 300])
+@pytest.mark.parametrize("rows,n", [(1, 100), (3, 5000), (1, 262145), (12, 65536), (13, 65536),
+                                    (300, 5377), (400, 6001)])
+def test_mfma_strips_by_size(hip, K, rows, n):
+    """The strip does not change a bit of the result."""
+    import torch
+    from scir_amd import device
+    L = hip.lib()
+    print(f"strips by size [{rows},{n}] K={K}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(K + n)
+    x = torch.randn((rows, n), device="cuda", generator=g)
+    b = torch.randn((K,), device="cuda", generator=g)
+    if rows * n * ((K + 14) // 16 + 1) >= 1 << 24:
+        pytest.skip("not on the FP32 matrix cores")
+    y, dx = device.fir(x, b, "f32"), device.vjp_dx(x, b, "f32")
+    try:
+        hip.check(L.scir_hip_tune_set(b"direct.mfma_strip", 64))
+        assert torch.equal(y, device.fir(x, b, "f32"))
+        assert torch.equal(dx, device.vjp_dx(x, b, "f32"))
+    finally:
+        hip.check(L.scir_hip_tune_set(b"direct.mfma_strip", -1))

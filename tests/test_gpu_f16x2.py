@@ -104,6 +104,22 @@ def test_taken_from_its_size_up_matches_fp32_matrix_cores(hip, oracle):
     assert np.all(np.abs(y - y64) <= lim) and np.all(np.abs(y32 - y64) <= lim)
 
 
+def test_long_segments_of_many_rows(hip, oracle):
+    """Rows enough that the segments are of 8192 samples (test_segment_edges
+    has the short ones): one, and one sample into the second."""
+    import torch
+    from scir_amd import device
+    r = rng(8)
+    for rows, N in ((513, 8192), (300, 8193)):
+        print(f"f16x2 long segments [{rows},{N}]", flush=True)
+        x = r.standard_normal((rows, N)).astype(np.float32)
+        b = r.standard_normal(514).astype(np.float32)
+        y = device.fir(torch.tensor(x, device="cuda"), torch.tensor(b, device="cuda"), "f32")
+        keep = [0, 1, rows // 2, rows - 1]
+        y = y.cpu().numpy()[keep].astype(np.float64)
+        assert np.all(np.abs(y - oracle.lfilter_f64(x[keep], b)) <= bound(oracle, x[keep], b))
+
+
 def test_ragged_filters_of_every_length(hip, oracle):
     """One batch with filters from 0 to 1500 taps (below 16: BF16x3), with
     the work (a long signal) that makes its F32 plan take this path."""
