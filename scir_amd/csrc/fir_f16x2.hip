@@ -31,16 +31,21 @@
 //   * every nonzero |X| >= 2^-T with T = 10 + floor(log2(K + 1)) (its floor of
 //     2^-36 is at most (K+1) 2^-26 of its term), and
 //   * taps below 2^-14 (the zero crossings of a sinc come out as 1e-17, not
-//     as 0), whose errors are at most err = sum min(|B|, 2^-35), cannot carry
-//     an output alone: no sample of the window is zero, and max |X| / min |X|
-//     <= ratio, which bounds err max|X| by (K+1) 2^-25 min|X| sum|B|, so by
-//     (K+1) 2^-25 sum |B||X| (at the row start, where outputs see the first
-//     taps alone: for every prefix of the taps).
-// A segment outside these limits (and every segment of a filter of fewer than
-// 16 taps, where the bound leaves no room, or of one with an Inf) is filtered
-// by the BF16x3 contraction in the same workgroup, half a segment at a time.
-// The choice and the scale depend on the segment's samples and the taps alone,
-// so the result does not depend on how segments are grouped.
+//     as 0), whose errors are at most err = sum min(|B|, 2^-35), do not carry
+//     an output alone.  They do not where |Y| >= 2 err max|X| / ((K+1) 2^-25),
+//     for |Y| is a lower bound of sum |B||X| (up to the errors, hence the 2):
+//     about 1e-9 of full scale.  Of smaller outputs, the row's first 16 (a
+//     first tap that is almost zero) are recomputed from the reference loop's
+//     terms, those that see zeros only are exact, and a segment with others
+//     (impulses in silence) is filtered again by BF16x3.  (Ruling such
+//     segments out from the samples' and the taps' magnitudes instead sent
+//     every segment with a zero sample to BF16x3: ten zeros in 67 million
+//     samples cost 37 of 370 us.)
+// A segment outside the first limit (and every segment of a filter of fewer
+// than 16 taps, where the bound leaves no room, or of one with an Inf) is
+// filtered by the BF16x3 contraction in the same workgroup, half a segment at
+// a time.  The choice and the scale depend on the segment's samples and the
+// taps alone, so the result does not depend on how segments are grouped.
 #include "toeplitz_mfma.hpp"
 
 namespace scir {
@@ -52,14 +57,12 @@ constexpr int kMaxTaps = 2049;    // history units fit the prefetched ones (m_hi
 // Words of LDS the waves exchange: per wave (4) unless said otherwise.
 enum Word {
     kSampleMax = 0,    // |x| bits, of the next segment to stage
-    kSampleMin = 4,
-    kSampleExp = 8,    // smallest exponent of a nonzero sample
-    kTapSum = 12,      // sum of |B|
-    kTapErr = 16,      // bound of the errors of the taps below 2^-14
-    kTapMax = 20,      // |b| bits
-    kTapRatio = 24,    // smallest sum / error over the taps' prefixes
-    kMins3 = 28,       // 8 words: the BF16x3 path's exponents
-    kWords = 36
+    kSampleExp = 4,    // smallest exponent of a nonzero sample
+    kTapErr = 8,       // bound of the errors of the taps below 2^-14
+    kTapMax = 12,      // |b| bits
+    kRedo = 16,        // the wave has doubtful outputs
+    kMins3 = 20,       // 8 words: the BF16x3 path's exponents
+    kWords = 28
 };
 
 // LDS: two split arrays of a segment (or three of half a segment), the tap
@@ -108,13 +111,6 @@ __device__ __forceinline__ float uniform(float v)
     return __builtin_bit_cast(float, uniform(__builtin_bit_cast(int, v)));
 }
 
-// min(a, |b|, |c|), NaN if any is: one v_minimum3_f32.
-__device__ __forceinline__ float minimum3(float a, float b, float c)
-{
-    return __builtin_elementwise_minimum(
-        __builtin_elementwise_minimum(__builtin_fabsf(b), __builtin_fabsf(c)), a);
-}
-
 // Scale exponent that puts a largest magnitude (bits mx) in [2^13, 2^14).
 __device__ __forceinline__ int scale_exponent(unsigned int mx)
 {
@@ -156,8 +152,9 @@ struct SplitGroup {
     const float *b;
     int K, m_hi;
     int sx, sb, T;
-    bool always3, tiny_taps;
-    float ratio, ratio_start;  // of segments inside the row, and at its start
+    bool always3;
+    float doubt;  // scaled outputs below it may hang on the taps below 2^-14; or 0
+    bool zeros;   // the segment last measured
     Table table;
 
     __device__ __forceinline__ int *words() const
@@ -174,14 +171,11 @@ struct SplitGroup {
         table = kTwo;
     }
 
-    // Notes the magnitudes of the segment in `raw` (first sample xb of a row of
-    // N) in this wave's words, for the scale and the choice that every wave
-    // makes after the next barrier.  Zeros outside the row do not count.
-    __device__ __forceinline__ void measure(const f32x4 (&raw)[PF][2], int64_t N, int64_t xb,
-                                            int tid)
+    // Notes the magnitudes of the segment in `raw` in this wave's words, for
+    // the scale and the choice that every wave makes after the next barrier.
+    __device__ __forceinline__ void measure(const f32x4 (&raw)[PF][2], int tid)
     {
         float largest = 0.0f, least = __builtin_inff();  // NaN once there is one
-        unsigned int mn;
         const int n = units();
 #pragma unroll
         for (int j = 0; j < PF; ++j) {
@@ -193,41 +187,29 @@ struct SplitGroup {
             }
         }
         const int wmx = wave_umax(abs_bits(largest));
-        int wmn = wave_umin(abs_bits(least)), we;
-        if (wmn != 0) {
-            we = __builtin_amdgcn_frexp_expf(__builtin_bit_cast(float, wmn));
-        } else {
-            // A zero: outside the row, or the smallest nonzero magnitude is
-            // another.
-            int e = 0;
-            mn = 0x7fffffffu;
+        unsigned int wmn = (unsigned)wave_umin(abs_bits(least));
+        if (wmn == 0) {  // the smallest nonzero one: zeros wrap round
+            unsigned int mn = 0xffffffffu;
 #pragma unroll
             for (int j = 0; j < PF; ++j) {
-                const int u = tid + j * kThreads;
-                if (u >= n) break;
-                const int64_t g0 = xb + 8 * (int64_t)u;
+                if (tid + j * kThreads >= n) break;
 #pragma unroll
-                for (int c = 0; c < 8; ++c) {
-                    const float v = unit_sample<REV>(raw[j], c);
-                    e = min_exponent(e, v);
-                    if (g0 + c >= 0 && g0 + c < N) mn = min(mn, abs_bits(v));
-                }
+                for (int c = 0; c < 8; ++c) mn = min(mn, abs_bits(raw[j][c >> 2][c & 3]) - 1);
             }
-            wmn = wave_umin(mn);
-            we = wave_min(e);
+            wmn = (unsigned)wave_umin(mn) + 1;
         }
         if ((tid & 63) == 0) {
             int *w = words() + (tid >> 6);
             w[kSampleMax] = wmx;
-            w[kSampleMin] = wmn;
-            w[kSampleExp] = we;
+            w[kSampleExp] =
+                wmn ? __builtin_amdgcn_frexp_expf(__builtin_bit_cast(float, wmn)) : 128;
         }
     }
 
     // Takes a filter and the first segment it is for (in `raw`).  The LDS is
     // free on entry and on return; barriers inside.
     __device__ __forceinline__ void begin(const float *taps, int ntaps, bool same_filter,
-                                          const f32x4 (&raw)[PF][2], int64_t N, int64_t P0)
+                                          const f32x4 (&raw)[PF][2])
     {
         // Opaque, so that nothing derived from it is kept in registers across
         // the work items of the ragged kernel.
@@ -254,7 +236,7 @@ struct SplitGroup {
             m = (unsigned)wave_umax(m);
             if (lane == 0) w[kTapMax + wave] = (int)m;
         }
-        measure(raw, N, 32 * P0 - 16 * (int64_t)m_hi, tid);
+        measure(raw, tid);
         __syncthreads();
         if (same_filter) return;
         const unsigned int b_max = (unsigned)uniform(
@@ -263,77 +245,37 @@ struct SplitGroup {
         sb = b_max < 0x7f800000u ? uniform(scale_exponent(b_max)) : 0;
         always3 = K < kMinTaps || b_max >= 0x7f800000u || sb < -100 || sb > 100;
         T = 10 + 31 - __builtin_clz(K + 1);
-        tiny_taps = false;
+        doubt = 0.0f;
         table = kNone;
         if (always3) return;
-        // Sums of |B| and of the tiny taps' errors: the thread's own, then over
-        // the lanes before it, then over the waves.
-        float sum = 0.0f, err = 0.0f;
-        auto add = [&](float tap) {
-            const float a = __builtin_fabsf(tap * pow2(sb));
-            const bool tiny = tap != 0.0f && a < 0x1p-14f;
-            sum += a;
-            err += tiny ? fmaxf(fminf(a, 0x1p-35f), 0x1p-149f) : 0.0f;
-            return tiny;
-        };
+        float err = 0.0f;
 #pragma unroll
-        for (int r = 0; r < kRun; ++r) add(v[r]);
+        for (int r = 0; r < kRun; ++r) {
+            const float a = __builtin_fabsf(v[r] * pow2(sb));
+            if (v[r] != 0.0f && a < 0x1p-14f) err += fmaxf(fminf(a, 0x1p-35f), 0x1p-149f);
+        }
 #pragma unroll
-        for (int d = 1; d < 64; d <<= 1) {
-            const float s2 = __shfl_up(sum, d, 64), e2 = __shfl_up(err, d, 64);
-            if (lane >= d) {
-                sum += s2;
-                err += e2;
-            }
-        }
-        if (lane == 63) {
-            w[kTapSum + wave] = __builtin_bit_cast(int, sum);
-            w[kTapErr + wave] = __builtin_bit_cast(int, err);
-        }
-        const float sum_before = __shfl_up(sum, 1, 64), err_before = __shfl_up(err, 1, 64);
+        for (int d = 32; d >= 1; d >>= 1) err += __shfl_xor(err, d, 64);
+        if (lane == 0) w[kTapErr + wave] = __builtin_bit_cast(int, err);
         build_two();
         __syncthreads();
-        auto shared = [&](int at, int n) {
-            float s = 0.0f;
-            for (int i = 0; i < n; ++i) s += __builtin_bit_cast(float, w[at + i]);
-            return s;
-        };
-        const float total_err = shared(kTapErr, 4), slack = (float)(K + 1) * 0x1p-25f;
-        tiny_taps = uniform((int)(total_err > 0.0f)) != 0;
-        if (!tiny_taps) return;
-        ratio = uniform(shared(kTapSum, 4) * slack / total_err);
-        sum = shared(kTapSum, wave) + (lane ? sum_before : 0.0f);
-        err = shared(kTapErr, wave) + (lane ? err_before : 0.0f);
-        float least = __builtin_inff();
-#pragma unroll
-        for (int r = 0; r < kRun; ++r)
-            if (add(v[r])) least = fminf(least, sum / err);
-        // Half of it: the sums' own rounding.
-        const int wl = wave_umin(__builtin_bit_cast(unsigned int, least * 0.5f));
-        if (lane == 0) w[kTapRatio + wave] = wl;
-        __syncthreads();
-        ratio_start = uniform(slack * __builtin_bit_cast(float,
-            (int)min(min((unsigned)w[kTapRatio], (unsigned)w[kTapRatio + 1]),
-                     min((unsigned)w[kTapRatio + 2], (unsigned)w[kTapRatio + 3]))));
+        err = 0.0f;
+        for (int i = 0; i < 4; ++i) err += __builtin_bit_cast(float, w[kTapErr + i]);
+        // 2 err max|X| / ((K + 1) 2^-25), max|X| < 2^14.
+        doubt = uniform(err * 0x1p+40f / (float)(K + 1));
     }
 
     // Whether the segment last measured fits the split, and its scale.
-    __device__ __forceinline__ bool fit(bool at_start)
+    __device__ __forceinline__ bool fit()
     {
         const int *w = words();
         const unsigned int mx = (unsigned)uniform((int)max(
             max((unsigned)w[0], (unsigned)w[1]), max((unsigned)w[2], (unsigned)w[3])));
-        const unsigned int mn = (unsigned)uniform((int)min(
-            min((unsigned)w[kSampleMin], (unsigned)w[kSampleMin + 1]),
-            min((unsigned)w[kSampleMin + 2], (unsigned)w[kSampleMin + 3])));
         const int e = uniform(min(min(w[kSampleExp], w[kSampleExp + 1]),
                                   min(w[kSampleExp + 2], w[kSampleExp + 3])));
         sx = uniform(scale_exponent(mx));
+        zeros = mx == 0;
         if (always3 || mx >= 0x7f800000u || sx < -100 || sx > 100) return false;
-        if (tiny_taps &&
-            (mn == 0 || __builtin_bit_cast(float, mx) > (at_start ? ratio_start : ratio) *
-                                                            __builtin_bit_cast(float, mn)))
-            return false;
         return e >= 1 - T - sx;
     }
 
@@ -384,7 +326,7 @@ struct SplitGroup {
                                             int tid, Next next)
     {
         const int wave = tid >> 6, lane = tid & 63;
-        const bool two = fit(P0 < (m_hi + 1) / 2);
+        const bool two = fit();
         if (two) {
             if (table != kTwo) build_two();
             const SplitScale scale = split_scale(sx);
@@ -399,16 +341,26 @@ struct SplitGroup {
         next();
         if (two) {
             // A wave past the row end has no output (see fir_mfma_kernel).
+            bool more = false;
             if (32 * (P0 + (int64_t)uniform(wave) * 32 * TW) < N) {
                 const int i = lane & 31, g = lane >> 5;
                 Contraction<2, TW> ct;
                 contract_segment<2, TW>(ct, lds, lay.stride2, lay.tab_offset, lay.copy2,
                                         m_hi + 2, m_hi, wave, i, g);
                 wait_for_loads();
-                store_segment<2, TW, REV>(ct, yrow, N, P0, wave, i, g, xrow, b, K, false,
-                                          -(sx + sb));
+                const int e = -(sx + sb);
+                const float d = doubt > 0.0f && !zeros ? __builtin_ldexpf(doubt, e) + 0x1p-149f
+                                                       : 0.0f;
+                const SplitOutputs so = {e, d, m_hi};
+                more = store_segment<2, TW, REV>(ct, yrow, N, P0, wave, i, g, xrow, b, K, false,
+                                                 so);
             }
-            return;
+            if (doubt == 0.0f || zeros) return;
+            int *w = words() + kRedo;
+            const bool any = __any(more);
+            if (lane == 0) w[wave] = any;
+            __syncthreads();
+            if (!uniform(w[0] | w[1] | w[2] | w[3])) return;
         }
 #pragma unroll 1
         for (int h = 0; h < TW; ++h)
@@ -446,7 +398,7 @@ __global__ __launch_bounds__(kThreads, 2) void fir_f16x2_kernel(
     Group group;
     group.lds = lds;
     group.lay = lay;
-    group.begin(b, K, false, raw, N, (int64_t)seg * Group::SEG_BLOCKS);
+    group.begin(b, K, false, raw);
     for (int done = 0; done < count; ++done) {
         // Lane-dependent values are recomputed in every iteration (see
         // fir_mfma_kernel).
@@ -454,7 +406,7 @@ __global__ __launch_bounds__(kThreads, 2) void fir_f16x2_kernel(
         asm volatile("" : "+v"(tid));
         const int64_t P0 = (int64_t)seg * Group::SEG_BLOCKS;
         if (done) {
-            group.measure(raw, N, 32 * P0 - 16 * (int64_t)m_hi, tid);
+            group.measure(raw, tid);
             __syncthreads();  // the previous segment's MFMAs are done
         }
         const bool last = seg + 1 == segs_per_row;
@@ -507,15 +459,14 @@ __global__ __launch_bounds__(kThreads, 2) void fir_f16x2_ragged_kernel(
         if (threadIdx.x == 0) s_item[parity] = (int)atomicAdd(counter, 1u);
         __syncthreads();  // every wave is done with the previous item's LDS; slot written
         nxt = uniform(s_item[parity]);
-        group.begin(b + w.b0, w.K, b + w.b0 == group.b && w.K == group.K, raw, w.len,
-                    (int64_t)w.seg0 * Group::SEG_BLOCKS);
+        group.begin(b + w.b0, w.K, b + w.b0 == group.b && w.K == group.K, raw);
         const int64_t seg_end = (int64_t)w.seg0 + w.nseg;
         for (int64_t sg = w.seg0; sg < seg_end; ++sg) {
             int tid = (int)threadIdx.x;
             asm volatile("" : "+v"(tid));
             const int64_t P0 = sg * Group::SEG_BLOCKS;
             if (sg != w.seg0) {
-                group.measure(raw, w.len, 32 * P0 - 16 * (int64_t)group.m_hi, tid);
+                group.measure(raw, tid);
                 __syncthreads();  // the previous segment's MFMAs are done
             }
             group.segment(raw, x + w.x0, y + w.x0, w.len, P0, tid, [&] {

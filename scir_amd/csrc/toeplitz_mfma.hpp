@@ -249,6 +249,13 @@ __device__ __forceinline__ float maximum3(float a, float b, float c)
         __builtin_elementwise_maximum(__builtin_fabsf(b), __builtin_fabsf(c)), a);
 }
 
+// min(a, |b|, |c|), NaN if any is: one v_minimum3_f32.
+__device__ __forceinline__ float minimum3(float a, float b, float c)
+{
+    return __builtin_elementwise_minimum(
+        __builtin_elementwise_minimum(__builtin_fabsf(b), __builtin_fabsf(c)), a);
+}
+
 template <int S>
 __device__ __forceinline__ f32x16 mfma(u32x4 a, u32x4 b, f32x16 c)
 {
@@ -665,30 +672,66 @@ __device__ __forceinline__ void contract_segment(Contraction<S, TW> &ct, const u
 // contraction.
 __device__ __forceinline__ void wait_for_loads() { __builtin_amdgcn_s_waitcnt(0x0f70); }
 
+// What F16x2 adds to a segment's epilogue.
+struct SplitOutputs {
+    int out_exp = 0;      // the operands' scale, taken back
+    float doubt = 0.0f;   // smaller outputs may hang on taps the split has lost
+    int m_hi = 0;
+};
+
+// Whether the 32 outputs of the workgroup's block `p` see zeros only: their
+// staged samples (units from 4p on: the history, then the block).  Nonzero
+// samples have a nonzero high term (fir_f16x2.hip's range).
+template <int TW>
+__device__ __forceinline__ bool silent_block(const unsigned char *lds, int p, int m_hi)
+{
+    const int end = 4 * p + 2 * m_hi + 4;
+#pragma unroll 1
+    for (int u = 4 * p; u < end; u += 8) {
+        unsigned int any = 0;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {  // past the end: the last unit again
+            const u32x4 w =
+                *reinterpret_cast<const u32x4 *>(lds + unit_addr<TW>(min(u + k, end - 1)));
+            any |= w.x | w.y | w.z | w.w;
+        }
+        if (any & 0x7fff7fffu) return false;
+    }
+    return true;
+}
+
 // Epilogue: tile t, lane (i, g) holds block P0 + wave*32*TW + t + TW*i,
 // samples 8q + 4g + j; outputs past N are dropped.  A non-finite output, and
 // every output of a segment with tiny magnitudes, is recomputed from the
-// reference loop's terms (x row xrow, taps b[0, K)).
+// reference loop's terms (x row xrow, taps b[0, K)).  So is a doubtful one
+// (F16x2) among the row's first 16; returns whether the lane has another that
+// is not an exact zero of a silent block.
 template <int S, int TW, bool REV>
-__device__ __forceinline__ void store_segment(const Contraction<S, TW> &ct,
+__device__ __forceinline__ bool store_segment(const Contraction<S, TW> &ct,
                                               float *__restrict__ yrow, int64_t N, int64_t P0,
                                               int wave, int i, int g,
                                               const float *__restrict__ xrow,
                                               const float *__restrict__ b, int K, bool tiny,
-                                              int out_exp = 0)
+                                              const SplitOutputs &so = {})
 {
-    // F16x2: back from the scale of the split operands (a power of two).
     auto output = [&](int t, int e) {
         const float v = ct.output(t, e);
-        return S == 2 ? __builtin_ldexpf(v, out_exp) : v;
+        return S == 2 ? __builtin_ldexpf(v, so.out_exp) : v;
     };
-    // Every output of the wave inside the row (a wave-uniform test): the
-    // stores go out unconditionally, half an instruction per output notes a
-    // non-finite one, and only such (or tiny) segment runs the recomputation pass over
-    // the stored values (rolled loops: indexing the accumulators there would
-    // put them in scratch).
-    if (32 * (P0 + (int64_t)(wave + 1) * 32 * TW) <= N) {
-        float largest = 0.0f;  // NaN once there is one
+    // Half an instruction per output notes a non-finite one, and half a
+    // doubtful one; only such (or a tiny segment) runs a second pass.
+    float largest = 0.0f;  // NaN once there is one
+    float least[TW], least_head = __builtin_inff();  // a tile's; its first 8 samples of t = 0
+    auto note = [&](int t, int q, const f32x4 &v) {
+        largest = maximum3(maximum3(largest, v.x, v.y), v.z, v.w);
+        if (S != 2) return;
+        float &l = t == 0 && q < 2 ? least_head : least[t];
+        l = minimum3(minimum3(l, v.x, v.y), v.z, v.w);
+    };
+    const bool whole = 32 * (P0 + (int64_t)(wave + 1) * 32 * TW) <= N;  // wave-uniform
+#pragma unroll
+    for (int t = 0; t < TW; ++t) least[t] = __builtin_inff();
+    if (whole) {
 #pragma unroll
         for (int t = 0; t < TW; ++t) {
             const int64_t n0 = 32 * (P0 + wave * 32 * TW + t + TW * i) + 4 * g;
@@ -697,7 +740,7 @@ __device__ __forceinline__ void store_segment(const Contraction<S, TW> &ct,
                 f32x4 v;
 #pragma unroll
                 for (int j = 0; j < 4; ++j) v[j] = output(t, 4 * q + j);
-                largest = maximum3(maximum3(largest, v.x, v.y), v.z, v.w);
+                note(t, q, v);
                 const int64_t n = n0 + 8 * q;
                 if (!REV)
                     *reinterpret_cast<f32x4u *>(yrow + n) = v;
@@ -705,53 +748,74 @@ __device__ __forceinline__ void store_segment(const Contraction<S, TW> &ct,
                     *reinterpret_cast<f32x4u *>(yrow + (N - 4 - n)) = f32x4{v.w, v.z, v.y, v.x};
             }
         }
-        if (tiny || !__builtin_isfinite(largest)) {
-#pragma unroll 1
-            for (int t = 0; t < TW; ++t) {
-                const int64_t n0 = 32 * (P0 + wave * 32 * TW + t + TW * i) + 4 * g;
-#pragma unroll 1
-                for (int q = 0; q < 4; ++q) {
-                    const int64_t n = n0 + 8 * q;
-#pragma unroll 1
-                    for (int j = 0; j < 4; ++j) {
-                        // The thread's own store above, read back.
-                        float &y = yrow[REV ? N - 1 - (n + j) : n + j];
-                        if (tiny || !__builtin_isfinite(y))
-                            y = direct_output<false>(xrow, N, REV, b, K, n + j);
-                    }
+    } else {
+#pragma unroll
+        for (int t = 0; t < TW; ++t) {
+            const int64_t n0 = 32 * (P0 + wave * 32 * TW + t + TW * i) + 4 * g;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int64_t n = n0 + 8 * q;
+                f32x4 v;
+#pragma unroll
+                for (int j = 0; j < 4; ++j) v[j] = output(t, 4 * q + j);
+                if (n + 3 < N) {
+                    note(t, q, v);
+                    if (!REV)
+                        *reinterpret_cast<f32x4u *>(yrow + n) = v;
+                    else
+                        *reinterpret_cast<f32x4u *>(yrow + (N - 4 - n)) =
+                            f32x4{v.w, v.z, v.y, v.x};
+                } else {
+#pragma unroll
+                    for (int j = 0; j < 4; ++j)
+                        if (n + j < N) {
+                            note(t, q, f32x4{v[j], v[j], v[j], v[j]});
+                            yrow[REV ? N - 1 - (n + j) : n + j] = v[j];
+                        }
                 }
             }
         }
-        return;
     }
-#pragma unroll
-    for (int t = 0; t < TW; ++t) {
-        const int64_t n0 = 32 * (P0 + wave * 32 * TW + t + TW * i) + 4 * g;
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            f32x4 v;
-#pragma unroll
-            for (int j = 0; j < 4; ++j) v[j] = output(t, 4 * q + j);
-            const int64_t n = n0 + 8 * q;
-            if (tiny || !__builtin_isfinite(v.x) || !__builtin_isfinite(v.y) ||
-                !__builtin_isfinite(v.z) || !__builtin_isfinite(v.w)) {
-#pragma unroll
-                for (int j = 0; j < 4; ++j)
-                    if (n + j < N && (tiny || !__builtin_isfinite(v[j])))
-                        v[j] = direct_output<false>(xrow, N, REV, b, K, n + j);
-            }
-            if (n + 3 < N) {
-                if (!REV)
-                    *reinterpret_cast<f32x4u *>(yrow + n) = v;
-                else
-                    *reinterpret_cast<f32x4u *>(yrow + (N - 4 - n)) = f32x4{v.w, v.z, v.y, v.x};
-            } else {
-#pragma unroll
-                for (int j = 0; j < 4; ++j)
-                    if (n + j < N) yrow[REV ? N - 1 - (n + j) : n + j] = v[j];
+    if (tiny || !__builtin_isfinite(largest)) {
+        // Over the stored values, in rolled loops: indexing the accumulators
+        // there would put them in scratch.
+#pragma unroll 1
+        for (int t = 0; t < TW; ++t) {
+            const int64_t n0 = 32 * (P0 + wave * 32 * TW + t + TW * i) + 4 * g;
+#pragma unroll 1
+            for (int e = 0; e < 16; ++e) {
+                const int64_t n = n0 + 8 * (e >> 2) + (e & 3);
+                if (n >= N) break;
+                // The thread's own store above, read back.
+                float &y = yrow[REV ? N - 1 - n : n];
+                if (tiny || !__builtin_isfinite(y))
+                    y = direct_output<false>(xrow, N, REV, b, K, n);
             }
         }
     }
+    bool more = false;
+    if (S == 2 && so.doubt > 0.0f) {
+        const bool head = P0 == 0 && wave == 0 && i == 0;
+        if (head && least_head < so.doubt) {
+            unsigned int which = 0;
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+                which |= __builtin_fabsf(output(0, e)) < so.doubt ? 1u << e : 0u;
+#pragma unroll 1
+            for (; which; which &= which - 1) {
+                const int e = __builtin_ctz(which);
+                const int64_t n = 8 * (e >> 2) + 4 * g + (e & 3);
+                if (n < N)
+                    yrow[REV ? N - 1 - n : n] = direct_output<false>(xrow, N, REV, b, K, n);
+            }
+        }
+        if (!head) least[0] = fminf(least[0], least_head);
+#pragma unroll
+        for (int t = 0; t < TW; ++t)
+            if (least[t] < so.doubt)
+                more |= !silent_block<TW>(ct.lds, wave * 32 * TW + t + TW * i, so.m_hi);
+    }
+    return more;
 }
 
 }  // namespace

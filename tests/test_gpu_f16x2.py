@@ -51,6 +51,29 @@ def sinc_with_zero_crossings(K):
     return b
 
 
+# Zero samples under taps that are almost zero: outputs that hang on one such
+# tap (at the row start, between impulses), silent stretches, zero rows.
+@pytest.mark.parametrize("K", [601, 1023])
+@pytest.mark.parametrize("what", ["quantised", "edges", "sparse", "zero_rows"])
+def test_zero_samples_and_almost_zero_taps(hip, oracle, K, what):
+    r = rng(K + len(what))
+    x = r.standard_normal((3, 20000)).astype(np.float32)
+    if what == "quantised":
+        x = np.round(x * 4).astype(np.float32)
+    elif what == "edges":
+        x[0, 300:9000] = 0.0
+        x[1, :8192] = 0.0
+        x[2, 4096:] = 0.0
+    elif what == "sparse":
+        x = np.where(np.arange(20000) % 2500 == 7, x, 0.0).astype(np.float32)
+    else:
+        x[:2] = 0.0
+        x[2, 1:] = 0.0
+    b = sinc_with_zero_crossings(K)
+    b[0] = np.float32(3e-17)
+    check(oracle, x, b, f"zeros {what}")
+
+
 @pytest.mark.parametrize("case", ["1e-30", "1e30", "1e-41", "ramp", "bursts", "impulses",
                                   "silence", "steps", "near_max"])
 @pytest.mark.parametrize("taps", ["random", "sinc", "decaying", "tiny"])
