@@ -413,17 +413,14 @@ __device__ __forceinline__ void collect_state(double (&z)[D], const double *zr, 
 // states, from zero state, of the outputs filtered back to front to
 // zs[rows*nC*2S + ...].  Bound by HBM (a RUN over 32 rows of 262144 moves
 // 134 MB in 27 us, the rate of a large copy) and, on short rows, by the
-// launches: butter(4) there as filtfilt 112 -> 86 us, as sosfilt 55 -> 48,
-// 64 rows of 9000 50 -> 31 and 25 -> 18.  The plan starts 4 waves a SIMD in
-// one go, so the collecting kernels are held to the 128 registers that
-// lets all of them run at once (four sections would spill).
-// REV runs each row back to front; chunk c is c-th in time, and back to
-// front the short chunk (when L does not divide N) comes first, so every
-// chunk starts at a multiple of L (16-byte aligned groups) and only the
-// first group in time can be short; every chunk after the first in time is
-// L long, so A^L is its transition.
+// launches: butter(4) there as filtfilt 112 -> 90 us, as sosfilt 55 -> 48,
+// 64 rows of 9000 50 -> 30 and 25 -> 18.  The plan starts 4 waves a SIMD in
+// one go, so the collecting kernels are held to the 128 registers that let
+// them run at once where that takes no scratch (not BACK, nor four sections:
+// three waves; a plan of three was slower, [1000, 65536] 589 -> 655 us).
 template <int SMAX, int MODE, bool REV, bool BACK = false>
-__global__ __launch_bounds__(kThreads, MODE == kCollect && SMAX <= 3 ? 4 : 1) void sos_wave_kernel(
+__global__ __launch_bounds__(kThreads, MODE == kCollect && !BACK && SMAX <= 3 ? 4 : 1) void
+sos_wave_kernel(
     const double *x, int64_t ldx, double *y, int64_t ldy, int64_t rows, int64_t N,
     const double *__restrict__ sos, int S, int64_t L, int64_t nC,
     const double *__restrict__ mats, double *__restrict__ zs, int vec)
