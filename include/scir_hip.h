@@ -381,7 +381,8 @@ SCIR_HIP_API int scir_hip_autotune_load(const char *cache_path);
  *   "mfma.tiles"      32x32 output tiles per wave of the MFMA kernel (1, 2, 4)
  *   "mfma.segs"       row segments per workgroup of the MFMA kernel (>= 1); the
  *                     next segment's samples load while the current one computes
- *   "vjp.db_mfma"     1 (default): dL/db on FP32 MFMA; 0: the FP32 VALU kernel
+ *   "vjp.db_mfma"     unset: dL/db by two fp16 terms on the 16-bit matrix
+ *                     cores; 1: on FP32 MFMA; 0: the FP32 VALU kernel
  *   "resample.fixed"  1 (default): up 2, down 3 with 31 taps (the reference's
  *                     only resample_poly case) runs the register-window
  *                     kernel; 0: the general polyphase kernel (same sums)

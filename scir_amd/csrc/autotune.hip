@@ -75,7 +75,10 @@ TuneChoice tune_lookup(int K, int64_t N)
     if (g_auto_fft_min_k >= 0) c.auto_fft_min_k = g_auto_fft_min_k;
     if (g_over_auto_fft >= 0) c.auto_fft = g_over_auto_fft != 0;
     if (g_over_auto_fft_min_k >= 0) c.auto_fft_min_k = g_over_auto_fft_min_k;
-    if (g_over_vjp_db_mfma >= 0) c.vjp_db_mfma = g_over_vjp_db_mfma != 0;
+    if (g_over_vjp_db_mfma >= 0) {
+        c.vjp_db_mfma = g_over_vjp_db_mfma != 0;
+        c.vjp_db_split = false;
+    }
     if (g_over_resample_fixed >= 0) c.resample_fixed = g_over_resample_fixed != 0;
     if (g_over_direct_r >= 0) c.direct_r = g_over_direct_r;
     if (g_over_direct_loader >= 0) c.direct_loader = g_over_direct_loader;

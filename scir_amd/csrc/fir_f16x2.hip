@@ -85,38 +85,6 @@ F16x2Layout f16x2_layout(int K, int tw)
 }
 inline size_t f16x2_lds(const F16x2Layout &l) { return (size_t)l.words_offset + 4 * kWords + 16; }
 
-__device__ __forceinline__ unsigned int abs_bits(float v)
-{
-    return __builtin_bit_cast(unsigned int, v) & 0x7fffffffu;
-}
-__device__ __forceinline__ float pow2(int e)  // |e| <= 126
-{
-    return __builtin_bit_cast(float, (unsigned int)(e + 127) << 23);
-}
-__device__ __forceinline__ SplitScale split_scale(int s)  // |s| <= 100
-{
-    return {pow2(s), pow2(-s), pow2(s + 11)};
-}
-__device__ __forceinline__ int wave_umax(unsigned int v)
-{
-    return wave_reduce((int)v, [](int a, int b) { return (int)max((unsigned)a, (unsigned)b); });
-}
-__device__ __forceinline__ int wave_umin(unsigned int v)
-{
-    return wave_reduce((int)v, [](int a, int b) { return (int)min((unsigned)a, (unsigned)b); });
-}
-__device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
-__device__ __forceinline__ float uniform(float v)
-{
-    return __builtin_bit_cast(float, uniform(__builtin_bit_cast(int, v)));
-}
-
-// Scale exponent that puts a largest magnitude (bits mx) in [2^13, 2^14).
-__device__ __forceinline__ int scale_exponent(unsigned int mx)
-{
-    return mx ? 14 - __builtin_amdgcn_frexp_expf(__builtin_bit_cast(float, mx)) : 0;
-}
-
 // Splits the 8 samples of unit u into the two split arrays.
 template <int TW, bool REV>
 __device__ __forceinline__ void store_unit2(unsigned char *lds, int stride, int u,

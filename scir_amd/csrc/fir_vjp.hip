@@ -8,9 +8,10 @@
 // N-1-i), so it reuses the dense direct/MFMA kernels through their `rev` mode
 // and inherits every precision mode.
 //
-// db is a correlation reduced over all rows and samples.  Stage 1 runs on
-// FP32 MFMA by default (fir_vjp_db_mfma_kernel, below); the tuning key
-// "vjp.db_mfma" = 0 selects the FP32 VALU form: a
+// db is a correlation reduced over all rows and samples.  Stage 1 runs by two
+// fp16 terms by default (fir_vjp_db_split_kernel, below); the tuning key
+// "vjp.db_mfma" = 1 selects FP32 MFMA (fir_vjp_db_mfma_kernel) and 0 the FP32
+// VALU form: a
 // workgroup walks `tiles_per_wg` tiles of T = 2048 samples of one row,
 // staging g and x (with K samples of history) in LDS.  Lane (kg, tg) owns 16
 // lags k0 + kg*16 + (0..15) and 128 samples tg*128 + (0..127) of a tile; it
@@ -20,14 +21,13 @@
 // partial[wg][k].  Stage 2 sums the partials over workgroups with Kahan
 // compensation in a fixed order.  Nothing is atomic: results are
 // deterministic.  Lags beyond 256 are handled in passes of 256.
-#include "common.hpp"
+#include "fp16_split.hpp"
 
 #include <algorithm>
 
 namespace scir {
 namespace {
 
-typedef float f32x4 __attribute__((ext_vector_type(4)));
 // Four floats at any 4-byte aligned global address (unaligned access mode).
 typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
 
@@ -142,6 +142,27 @@ __global__ __launch_bounds__(kThreads) void fir_vjp_db_partial_kernel(
 // order) and partial[wg][k] follow, which the final kernel reduces as before.
 constexpr int kMfmaLook = 256;  // g samples staged past the tile (16j + l < 256)
 
+// A wave's products of one tile (its samples m0 .. m0 + 511): four
+// accumulators in turn (independent MFMA chains of 32 products of 4 samples
+// each).  Sample group 4(4t + u) of the wave: each 16-sample step moves a
+// padded index by exactly 20 floats, so after the four bases the fully
+// unrolled loop's LDS reads carry constant offsets.
+__device__ __forceinline__ void db_products(const float *xs, const float *gs, int m0, int a_off,
+                                            int b_off, f32x4 &c0, f32x4 &c1, f32x4 &c2, f32x4 &c3)
+{
+    const float *xa0 = xs + pad16(m0 + a_off), *xa1 = xs + pad16(m0 + 4 + a_off);
+    const float *xa2 = xs + pad16(m0 + 8 + a_off), *xa3 = xs + pad16(m0 + 12 + a_off);
+    const float *gb0 = gs + pad16(m0 + b_off), *gb1 = gs + pad16(m0 + 4 + b_off);
+    const float *gb2 = gs + pad16(m0 + 8 + b_off), *gb3 = gs + pad16(m0 + 12 + b_off);
+#pragma unroll
+    for (int t = 0; t < kTile / 4 / 16; ++t) {  // 32 steps of 16 samples
+        c0 = __builtin_amdgcn_mfma_f32_16x16x4f32(xa0[20 * t], gb0[20 * t], c0, 0, 0, 0);
+        c1 = __builtin_amdgcn_mfma_f32_16x16x4f32(xa1[20 * t], gb1[20 * t], c1, 0, 0, 0);
+        c2 = __builtin_amdgcn_mfma_f32_16x16x4f32(xa2[20 * t], gb2[20 * t], c2, 0, 0, 0);
+        c3 = __builtin_amdgcn_mfma_f32_16x16x4f32(xa3[20 * t], gb3[20 * t], c3, 0, 0, 0);
+    }
+}
+
 __global__ __launch_bounds__(kThreads) void fir_vjp_db_mfma_kernel(
     const float *__restrict__ g, int64_t ldg, const float *__restrict__ x, int64_t ldx, int K,
     int64_t N, int segs_per_row, int tiles_per_wg, float *__restrict__ partial)
@@ -194,25 +215,223 @@ __global__ __launch_bounds__(kThreads) void fir_vjp_db_mfma_kernel(
             }
             __syncthreads();
             if (it + 1 < ntiles) fetch((tile0 + it + 1) * kTile, kp);
-            // Four accumulators in turn (independent MFMA chains of 32 products
-            // of 4 samples each per tile), added into the pass total per tile.
-            // Sample group 4(4t + u) of the wave: each 16-sample step moves a
-            // padded index by exactly 20 floats, so after the four bases the
-            // fully unrolled loop's LDS reads carry constant offsets.
-            const int m0 = 512 * wave;
-            const float *xa0 = xs + pad16(m0 + a_off), *xa1 = xs + pad16(m0 + 4 + a_off);
-            const float *xa2 = xs + pad16(m0 + 8 + a_off), *xa3 = xs + pad16(m0 + 12 + a_off);
-            const float *gb0 = gs + pad16(m0 + b_off), *gb1 = gs + pad16(m0 + 4 + b_off);
-            const float *gb2 = gs + pad16(m0 + 8 + b_off), *gb3 = gs + pad16(m0 + 12 + b_off);
             f32x4 c0 = {0.0f, 0.0f, 0.0f, 0.0f}, c1 = c0, c2 = c0, c3 = c0;
-#pragma unroll
-            for (int t = 0; t < kTile / 4 / 16; ++t) {  // 32 steps of 16 samples per wave
-                c0 = __builtin_amdgcn_mfma_f32_16x16x4f32(xa0[20 * t], gb0[20 * t], c0, 0, 0, 0);
-                c1 = __builtin_amdgcn_mfma_f32_16x16x4f32(xa1[20 * t], gb1[20 * t], c1, 0, 0, 0);
-                c2 = __builtin_amdgcn_mfma_f32_16x16x4f32(xa2[20 * t], gb2[20 * t], c2, 0, 0, 0);
-                c3 = __builtin_amdgcn_mfma_f32_16x16x4f32(xa3[20 * t], gb3[20 * t], c3, 0, 0, 0);
-            }
+            db_products(xs, gs, 512 * wave, a_off, b_off, c0, c1, c2, c3);
             tot += (c0 + c1) + (c2 + c3);
+        }
+        // C[i][j] in lane (j = li, i = 4 lq + v): lag kp + 4 lq + v + 16 li.
+#pragma unroll
+        for (int v = 0; v < 4; ++v) red[wave][4 * lq + v + 16 * li] = tot[v];
+        __syncthreads();
+        {
+            const int lag = kp + threadIdx.x;
+            const float sum = ((red[0][threadIdx.x] + red[1][threadIdx.x]) + red[2][threadIdx.x]) +
+                              red[3][threadIdx.x];
+            if (lag < K) partial[(int64_t)blockIdx.x * K + lag] = sum;
+        }
+        __syncthreads();  // red is rewritten by the next pass
+    }
+}
+
+// The same stage 1 by two fp16 terms (fp16_split.hpp) on
+// v_mfma_f32_16x16x32_f16: one product takes 32 samples against all 256 lags,
+//   C[i][j] += sum_l x[m + l - i - kp] * g[m + l + 16j],  l < 32,
+// as four (hi hi; hi lo and lo hi, at scale 2^11; lo lo, at 2^22: without it
+// sum x^2 is short by 5e-8), 64 matrix-core cycles where the FP32 form spends
+// 256.  Samples are split once per tile into LDS;
+// a lane's 8 consecutive g samples are 16-byte aligned, its x samples start
+// at any offset, so x is stored twice, the second copy one entry on, and a
+// lane reads the one where it is 4-byte aligned.  The tile's samples are
+// scaled by powers of two, which its sums take back before they are added to
+// the pass total.
+//
+// Sign: the matrix core's 16-bit products are summed with truncation towards
+// minus infinity, an error of one sign that a sum over millions of samples
+// collects (relative L2 2.1e-6 with outliers over 256 rows of 65536).  Every
+// other tile is therefore summed with -x, and subtracted: 1.6e-7, against
+// 2.1e-7 of the FP32 products.
+//
+// Range: a tile with an Inf, a NaN, or a nonzero sample below 2^-18 of the
+// scaled range (2^32 below the largest) runs by the FP32 products instead, so
+// every term is within 2^-17 of its magnitude, inside the sums' own bound,
+// (N/2048 + 200) 2^-24 sum|g||x|; almost every one within 2^-22.
+//
+// Bound by the LDS (both fragments of both operands for every four products).
+// [1024, 65536], K = 255: 309 us by the FP32 products, 245 by these (three
+// products, 230).
+constexpr int kDbMinExp = -17;  // frexp exponent of the smallest sample allowed (2^-18)
+
+__global__ __launch_bounds__(kThreads, 4) void fir_vjp_db_split_kernel(
+    const float *__restrict__ g, int64_t ldg, const float *__restrict__ x, int64_t ldx, int K,
+    int64_t N, int segs_per_row, int tiles_per_wg, float *__restrict__ partial)
+{
+    constexpr int GS = kTile + kMfmaLook;  // staged g samples
+    constexpr int XS = kTile + 32;         // staged x samples
+    // Bytes: g's terms; x's terms, two copies each (odd multiples of 128
+    // apart, so that even and odd lanes read different banks).
+    constexpr int GB = 2 * GS, XB = (2 * (XS + 8) + 255) / 256 * 256 + 128;
+    constexpr int kXBase = 2 * GB;
+    constexpr int kSplitBytes = kXBase + 4 * XB;
+    constexpr int kFloats = GS + GS / 4 + XS + XS / 4;  // the FP32 form's staging
+    constexpr int kBytes = kSplitBytes > 4 * kFloats ? kSplitBytes : 4 * kFloats;
+    __shared__ __attribute__((aligned(256))) unsigned char lds[kBytes];
+    __shared__ float red[kThreads / 64][kLagPass];
+    __shared__ int words[4][kThreads / 64];  // max of g, x; min exponents of g, x
+    float *gs = reinterpret_cast<float *>(lds), *xs = gs + GS + GS / 4;
+
+    const int64_t row = blockIdx.x / segs_per_row;
+    const int64_t tile0 = (int64_t)(blockIdx.x % segs_per_row) * tiles_per_wg;
+    const float *__restrict__ grow = g + row * ldg;
+    const float *__restrict__ xrow = x + row * ldx;
+    const int64_t tiles_in_row = (N + kTile - 1) / kTile;
+    const int ntiles = (int)min<int64_t>(tiles_per_wg, tiles_in_row - tile0);
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int li = lane & 15, lq = lane >> 4;
+
+    constexpr int NG = (GS / 4 + kThreads - 1) / kThreads, NX = (XS / 4 + kThreads - 1) / kThreads;
+    f32x4 pg[NG], px[NX];
+    auto fetch = [&](int64_t t0, int kp) {
+#pragma unroll
+        for (int u = 0; u < NG; ++u) {
+            const int v = threadIdx.x + u * kThreads;
+            pg[u] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            if (v < GS / 4) pg[u] = load4g(grow, t0 + 4 * v, N);
+        }
+#pragma unroll
+        for (int u = 0; u < NX; ++u) {
+            const int v = threadIdx.x + u * kThreads;
+            px[u] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            if (v < XS / 4) px[u] = load4g(xrow, t0 - kp - 16 + 4 * v, N);
+        }
+    };
+    // This wave's words of one operand.
+    auto measure = [&](const f32x4 *p, int n, int chunks, int which) {
+        float largest = 0.0f, least = __builtin_inff();  // NaN once there is one
+        for (int u = 0; u < n; ++u) {
+            if ((int)threadIdx.x + u * kThreads >= chunks) break;
+            largest = maximum3(maximum3(largest, p[u].x, p[u].y), p[u].z, p[u].w);
+            least = minimum3(minimum3(least, p[u].x, p[u].y), p[u].z, p[u].w);
+        }
+        const int mx = wave_umax(abs_bits(largest));
+        unsigned int mn = 0xffffffffu;  // the smallest nonzero one: zeros wrap round
+        if (wave_umin(abs_bits(least)) == 0) {
+            for (int u = 0; u < n; ++u) {
+                if ((int)threadIdx.x + u * kThreads >= chunks) break;
+                for (int c = 0; c < 4; ++c) mn = min(mn, abs_bits(p[u][c]) - 1);
+            }
+        } else {
+            mn = abs_bits(least) - 1;
+        }
+        mn = (unsigned)wave_umin(mn) + 1;  // 0: zeros only
+        if (lane == 0) {
+            words[which][wave] = mx;
+            words[2 + which][wave] =
+                mn ? __builtin_amdgcn_frexp_expf(__builtin_bit_cast(float, mn)) : 128;
+        }
+    };
+    // An operand's scale exponent, and whether its samples fit.
+    auto fit = [&](int which, int &s) {
+        const int *w = words[which], *e = words[2 + which];
+        const unsigned int mx = (unsigned)uniform(
+            (int)max(max((unsigned)w[0], (unsigned)w[1]), max((unsigned)w[2], (unsigned)w[3])));
+        s = uniform(scale_exponent(mx));
+        return mx < 0x7f800000u && s >= -100 && s <= 100 &&
+               uniform(min(min(e[0], e[1]), min(e[2], e[3]))) >= kDbMinExp - s;
+    };
+    for (int kp = 0; kp < K; kp += kLagPass) {
+        f32x4 tot = {0.0f, 0.0f, 0.0f, 0.0f};
+        fetch(tile0 * kTile, kp);
+        for (int it = 0; it < ntiles; ++it) {
+            measure(pg, NG, GS / 4, 0);
+            measure(px, NX, XS / 4, 1);
+            __syncthreads();  // words there, previous tile done with the LDS
+            int sg, sx;
+            const bool fit_g = fit(0, sg), fit_x = fit(1, sx);
+            const bool split = fit_g && fit_x;
+            const bool minus = (row + tile0 + it) & 1;
+            if (split) {
+                const SplitScale cg = split_scale(sg);
+                SplitScale cx = split_scale(sx);
+                if (minus) cx = {-cx.to, -cx.from, -cx.to_lo};
+#pragma unroll
+                for (int u = 0; u < NG; ++u) {
+                    const int v = threadIdx.x + u * kThreads;
+                    unsigned int h[2], l[2];
+                    split2_quad(pg[u], cg, h, l);
+                    if (v < GS / 4) {
+                        *reinterpret_cast<uint2 *>(lds + 8 * v) = make_uint2(h[0], h[1]);
+                        *reinterpret_cast<uint2 *>(lds + GB + 8 * v) = make_uint2(l[0], l[1]);
+                    }
+                }
+#pragma unroll
+                for (int u = 0; u < NX; ++u) {
+                    const int v = threadIdx.x + u * kThreads;
+                    unsigned int w[2][2];
+                    split2_quad(px[u], cx, w[0], w[1]);
+                    if (v < XS / 4) {
+#pragma unroll
+                        for (int t = 0; t < 2; ++t) {
+                            unsigned char *c0 = lds + kXBase + 2 * t * XB + 8 * v;
+                            *reinterpret_cast<uint2 *>(c0) = make_uint2(w[t][0], w[t][1]);
+                            unsigned char *c1 = c0 + XB + 2;  // one entry on
+                            *reinterpret_cast<unsigned short *>(c1) = (unsigned short)w[t][0];
+                            *reinterpret_cast<unsigned int *>(c1 + 2) =
+                                __builtin_amdgcn_alignbit(w[t][1], w[t][0], 16);
+                            *reinterpret_cast<unsigned short *>(c1 + 6) =
+                                (unsigned short)(w[t][1] >> 16);
+                        }
+                    }
+                }
+            } else {
+#pragma unroll
+                for (int u = 0; u < NG; ++u) {
+                    const int v = threadIdx.x + u * kThreads;
+                    if (v < GS / 4) *reinterpret_cast<f32x4 *>(gs + pad16(4 * v)) = pg[u];
+                }
+#pragma unroll
+                for (int u = 0; u < NX; ++u) {
+                    const int v = threadIdx.x + u * kThreads;
+                    if (v < XS / 4) *reinterpret_cast<f32x4 *>(xs + pad16(4 * v)) = px[u];
+                }
+            }
+            __syncthreads();
+            if (it + 1 < ntiles) fetch((tile0 + it + 1) * kTile, kp);
+            const int m0 = 512 * wave;
+            f32x4 c0 = {0.0f, 0.0f, 0.0f, 0.0f}, c1 = c0, c2 = c0, c3 = c0, c4 = c0;
+            if (split) {
+                // Lane (i = li, lq): x entries a .. a+7, a = m + 8 lq - i + 16;
+                // lane (j = li, lq): g entries m + 8 lq + 16 j + (0..7).
+                const int a = m0 + 8 * lq - li + 16, odd = a & 1;
+                const unsigned char *ax = lds + kXBase + odd * XB + 2 * (a + odd);
+                const unsigned char *bg = lds + 2 * (m0 + 8 * lq + 16 * li);
+#pragma unroll
+                for (int t = 0; t < kTile / 4 / 32; ++t) {  // 16 steps of 32 samples per wave
+                    u32x4 xh, xl;
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) {
+                        xh[c] = reinterpret_cast<const unsigned int *>(ax + 64 * t)[c];
+                        xl[c] = reinterpret_cast<const unsigned int *>(ax + 2 * XB + 64 * t)[c];
+                    }
+                    const f16x8 fh = __builtin_bit_cast(f16x8, xh);
+                    const f16x8 fl = __builtin_bit_cast(f16x8, xl);
+                    const f16x8 gh = *reinterpret_cast<const f16x8 *>(bg + 64 * t);
+                    const f16x8 gl = *reinterpret_cast<const f16x8 *>(bg + GB + 64 * t);
+                    f32x4 &hh = t & 1 ? c1 : c0;
+                    hh = __builtin_amdgcn_mfma_f32_16x16x32_f16(fh, gh, hh, 0, 0, 0);
+                    c2 = __builtin_amdgcn_mfma_f32_16x16x32_f16(fh, gl, c2, 0, 0, 0);
+                    c3 = __builtin_amdgcn_mfma_f32_16x16x32_f16(fl, gh, c3, 0, 0, 0);
+                    c4 = __builtin_amdgcn_mfma_f32_16x16x32_f16(fl, gl, c4, 0, 0, 0);
+                }
+                const f32x4 lo = c2 + (c3 + kLoUnscale * c4), hi = c0 + c1;
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    const float c = __builtin_fmaf(lo[v], kLoUnscale, hi[v]);
+                    tot[v] += __builtin_ldexpf(minus ? -c : c, -(sg + sx));
+                }
+            } else {
+                db_products(xs, gs, m0, 16 + lq - li, lq + 16 * li, c0, c1, c2, c3);
+                tot += (c0 + c1) + (c2 + c3);
+            }
         }
         // C[i][j] in lane (j = li, i = 4 lq + v): lag kp + 4 lq + v + 16 li.
 #pragma unroll
@@ -305,7 +524,7 @@ int vjp_db_args(const float *g, int64_t ldg, const float *x, int64_t ldx, int32_
 
 // dL/db on stream s (caller holds st->mu; arguments checked).  With `fixed`,
 // the partial sums go to that device buffer of `fixed_floats` floats instead
-// of the stream's library scratch (nothing is allocated): the FP32 MFMA
+// of the stream's library scratch (nothing is allocated): a matrix-core
 // stage 1 always runs, and when the usual workgroup count would not fit,
 // fewer workgroups per row walk longer runs of tiles.
 int vjp_db_run(const float *g, int64_t ldg, const float *x, int64_t ldx, int32_t K, int64_t B,
@@ -346,9 +565,15 @@ int vjp_db_run(const float *g, int64_t ldg, const float *x, int64_t ldx, int32_t
             SCIR_TRY(ensure_scratch(st, sc.partials, (size_t)nwg * K * sizeof(float), s));
             partial = static_cast<float *>(sc.partials.ptr);
         }
-        hipLaunchKernelGGL(fir_vjp_db_mfma_kernel, dim3((unsigned)nwg), dim3(kThreads), 0, s, g,
-                           ldg, x, ldx, (int)K, N, (int)segs, (int)tiles_per_wg, partial);
-        SCIR_TRY(check_launch("fir_vjp_db_mfma_kernel"));
+        // Below, both take the same time ([64, 4096], K = 255: 9.1 us); above,
+        // the split is the faster ([64, 16384]: 11.8 / 11.2, [64, 65536]: 31 / 25).
+        if (tc.vjp_db_split && B * N >= (int64_t)1 << 18)
+            hipLaunchKernelGGL(fir_vjp_db_split_kernel, dim3((unsigned)nwg), dim3(kThreads), 0, s,
+                               g, ldg, x, ldx, (int)K, N, (int)segs, (int)tiles_per_wg, partial);
+        else
+            hipLaunchKernelGGL(fir_vjp_db_mfma_kernel, dim3((unsigned)nwg), dim3(kThreads), 0, s,
+                               g, ldg, x, ldx, (int)K, N, (int)segs, (int)tiles_per_wg, partial);
+        SCIR_TRY(check_launch("dL/db stage 1"));
         hipLaunchKernelGGL(fir_vjp_db_final_kernel, dim3((K + kFinalLags - 1) / kFinalLags),
                            dim3(kThreads), 0, s, partial, nwg, (int)K, db);
         return check_launch("fir_vjp_db_final_kernel");

@@ -58,6 +58,7 @@
 #pragma once
 
 #include "direct_tiles.hpp"
+#include "fp16_split.hpp"
 
 #include <algorithm>
 
@@ -65,15 +66,12 @@ namespace scir {
 namespace {
 
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8;
-typedef __attribute__((__vector_size__(8 * sizeof(_Float16)))) _Float16 f16x8;
 typedef __attribute__((__vector_size__(16 * sizeof(float)))) float f32x16;
-typedef float f32x4 __attribute__((ext_vector_type(4)));
 // Four floats at any 4-byte aligned global address: the kernels load rows and
 // store outputs with 16-byte accesses whatever the row's offset or pitch (the
 // hardware runs in unaligned access mode; an access that crosses a cache line
 // costs two requests, far less than four 4-byte accesses).
 typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
-typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kWaves = 4;
 constexpr int kThreads = 64 * kWaves;
@@ -148,42 +146,6 @@ __device__ __forceinline__ void split3_pair(float v0, float v1, unsigned int &h,
     l = bf16x2_bits(r2);
 }
 
-typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
-constexpr float kLoUnscale = 1.0f / 2048.0f;  // 2^-11: the low term's scale is 2^11
-
-// The powers of two of an F16x2 split, of samples or taps.
-struct SplitScale {
-    float to;       // 2^s
-    float from;     // 2^-s
-    float to_lo;    // 2^(s + 11)
-};
-
-// The two fp16 terms, as packed words, of four values: three mixed-precision
-// multiply-adds a value (hi = rn(2^s v); v - 2^-s hi, exact; lo), where the
-// compiler's choice takes four and a half.  Each write of half a register is
-// one instruction away from the next use of that register, as the hardware
-// requires.
-__device__ __forceinline__ void split2_quad(const f32x4 &v, const SplitScale &c,
-                                            unsigned int (&h)[2], unsigned int (&l)[2])
-{
-    float r1, r3;
-    asm("v_fma_mixlo_f16 %0, %6, %10, 0\n\t"
-        "v_fma_mixlo_f16 %1, %8, %10, 0\n\t"
-        "v_fma_mixhi_f16 %0, %7, %10, 0\n\t"
-        "v_fma_mixhi_f16 %1, %9, %10, 0\n\t"
-        "v_fma_mix_f32 %2, %0, -%11, %6 op_sel_hi:[1,0,0]\n\t"
-        "v_fma_mix_f32 %4, %0, -%11, %7 op_sel:[1,0,0] op_sel_hi:[1,0,0]\n\t"
-        "v_fma_mix_f32 %3, %1, -%11, %8 op_sel_hi:[1,0,0]\n\t"
-        "v_fma_mix_f32 %5, %1, -%11, %9 op_sel:[1,0,0] op_sel_hi:[1,0,0]\n\t"
-        "v_fma_mixlo_f16 %2, %2, %12, 0\n\t"
-        "v_fma_mixlo_f16 %3, %3, %12, 0\n\t"
-        "v_fma_mixhi_f16 %2, %4, %12, 0\n\t"
-        "v_fma_mixhi_f16 %3, %5, %12, 0\n\t"
-        "s_nop 0"
-        : "=&v"(h[0]), "=&v"(h[1]), "=&v"(l[0]), "=&v"(l[1]), "=&v"(r1), "=&v"(r3)
-        : "v"(v.x), "v"(v.y), "v"(v.z), "v"(v.w), "s"(c.to), "s"(c.from), "s"(c.to_lo));
-}
-
 __device__ __forceinline__ unsigned int pack2(unsigned short lo, unsigned short hi)
 {
     return (unsigned int)lo | ((unsigned int)hi << 16);
@@ -202,19 +164,6 @@ __device__ __forceinline__ int min_exponent(int m, float v)
     return min(m, __builtin_amdgcn_frexp_expf(v));
 }
 
-// f over the wave (idempotent f: min or max): DPP row shifts, then row
-// broadcasts; all VALU.
-template <class F>
-__device__ __forceinline__ int wave_reduce(int v, F f)
-{
-    v = f(v, __builtin_amdgcn_update_dpp(v, v, 0x111, 0xF, 0xF, false));  // row_shr:1
-    v = f(v, __builtin_amdgcn_update_dpp(v, v, 0x112, 0xF, 0xF, false));  // row_shr:2
-    v = f(v, __builtin_amdgcn_update_dpp(v, v, 0x114, 0xF, 0xF, false));  // row_shr:4
-    v = f(v, __builtin_amdgcn_update_dpp(v, v, 0x118, 0xF, 0xF, false));  // row_shr:8
-    v = f(v, __builtin_amdgcn_update_dpp(v, v, 0x142, 0xA, 0xF, false));  // row_bcast:15
-    v = f(v, __builtin_amdgcn_update_dpp(v, v, 0x143, 0xC, 0xF, false));  // row_bcast:31
-    return __builtin_amdgcn_readlane(v, 63);
-}
 __device__ __forceinline__ int wave_min(int v)
 {
     return wave_reduce(v, [](int a, int b) { return min(a, b); });
@@ -240,20 +189,6 @@ __device__ __forceinline__ bool segment_is_tiny(const int *mins)
     const int ex = min(min(mins[0], mins[1]), min(mins[2], mins[3]));
     const int eb = min(min(mins[4], mins[5]), min(mins[6], mins[7]));
     return tiny_magnitudes(ex, eb);
-}
-
-// max(a, |b|, |c|), NaN if any is: one v_maximum3_f32.
-__device__ __forceinline__ float maximum3(float a, float b, float c)
-{
-    return __builtin_elementwise_maximum(
-        __builtin_elementwise_maximum(__builtin_fabsf(b), __builtin_fabsf(c)), a);
-}
-
-// min(a, |b|, |c|), NaN if any is: one v_minimum3_f32.
-__device__ __forceinline__ float minimum3(float a, float b, float c)
-{
-    return __builtin_elementwise_minimum(
-        __builtin_elementwise_minimum(__builtin_fabsf(b), __builtin_fabsf(c)), a);
 }
 
 template <int S>

@@ -79,6 +79,56 @@ def test_db_forms_vs_fp64(hip, oracle, B, N, K, mfma):
         hip.check(L.scir_hip_tune_set(b"vjp.db_mfma", -1))
 
 
+# The default form from 2^18 samples (two fp16 terms): tile edges (2048 samples,
+# 16 before, 256 past), passes of 256 lags, odd rows, samples that a scaled fp16 pair cannot
+# hold beside the largest (FP32 products), zero tiles, magnitudes far from 1.
+@pytest.mark.parametrize("what", ["normal", "1e-30", "1e-42", "1e18", "ramp", "zeros", "positive"])
+@pytest.mark.parametrize("B,N,K", [(17500, 15, 40), (130, 2047, 17), (128, 2048, 1),
+                                   (128, 2049, 256), (61, 4353, 257), (14, 20001, 513),
+                                   (1, 262147, 33)])
+def test_db_split_vs_fp64(hip, oracle, B, N, K, what):
+    print(f"dL/db by fp16 terms {what} [{B},{N}] K={K}", flush=True)
+    r = rng(B * 11 + N + K + len(what))
+    x = r.standard_normal((B, N)).astype(np.float32)
+    w = r.standard_normal((B, N)).astype(np.float32)
+    if what[0] == "1":
+        x = (x.astype(np.float64) * float(what)).astype(np.float32)
+    elif what == "ramp":
+        x = (x * 10.0 ** np.linspace(-15, 4, N)).astype(np.float32)
+        w = (w * 10.0 ** np.linspace(4, -15, N)).astype(np.float32)
+    elif what == "zeros":
+        x[:, N // 3:] = 0.0
+        w[:, ::7] = 0.0
+    elif what == "positive":
+        x, w = np.abs(x), np.abs(w)
+    b = np.zeros(K, np.float32)
+    _, db = gpu_grads(x, b, w)
+    _, db64 = oracle.vjp_f64(w, x, b)
+    bdb = bounds(oracle, x, b, w)[1] + B * N * 2.0 ** -149
+    assert np.all(np.abs(db - db64) <= bdb), f"db max excess {np.max(np.abs(db - db64) - bdb)}"
+
+
+def test_db_split_nonfinite(hip, oracle):
+    """Inf and NaN reach the lags that the FP32 products give them."""
+    import torch
+    from scir_amd import device
+    L = hip.lib()
+    r = rng(4)
+    x = torch.tensor(r.standard_normal((30, 9000)).astype(np.float32), device="cuda")
+    w = torch.tensor(r.standard_normal((30, 9000)).astype(np.float32), device="cuda")
+    x[0, 8990] = float("inf")
+    w[1, 100] = float("nan")
+    print("dL/db by fp16 terms, non-finite", flush=True)
+    db = device.vjp_db(w, x, 300)
+    try:
+        hip.check(L.scir_hip_tune_set(b"vjp.db_mfma", 1))
+        want = device.vjp_db(w, x, 300)
+    finally:
+        hip.check(L.scir_hip_tune_set(b"vjp.db_mfma", -1))
+    assert torch.equal(torch.isnan(db), torch.isnan(want))
+    assert torch.equal(torch.isinf(db), torch.isinf(want))
+
+
 def test_finite_differences(hip, oracle):
     """64 seeded coordinates (x and b), h = 1e-3, FP64 loss via the oracle."""
     r = rng(64)
