@@ -105,7 +105,7 @@ typedef enum scir_hip_precision {
     SCIR_HIP_PREC_FP16 = 3,
     /* Fastest of F32 / BF16X3 for the shape whose error is no larger (F32
      * below the cut-over of the autotuned table, 130 when none is loaded,
-     * and from K = 288 on large batches; F32 for K > 6689, beyond the MFMA
+     * and from K = 288 on batches of 2^25 outputs x K/16; F32 for K > 6689, beyond the MFMA
      * kernel's LDS); never FP16, and FFT32 only when the "auto.fft" key is set.  Either
      * choice keeps the F32 bound and the reference loop's non-finite
      * outputs, so AUTO is the drop-in default. */
@@ -371,11 +371,13 @@ SCIR_HIP_API int scir_hip_autotune_load(const char *cache_path);
  *                     (register prefetch), 2 = pipelined row segments copied
  *                     into LDS by DMA two tiles ahead (forward, 16-byte aligned
  *                     rows with N % 4 == 0; other calls use 1), 3 (default) =
- *                     F32 on FP32 MFMA for K <= 513 (F32_EXACT and longer
- *                     filters as 2)
- *   "direct.mfma_strip" 256-output tiles per wave of loader 3 (1 .. 4096;
- *                     default 4 for K <= 8, 8 to K = 40, 16 to K = 56, 32 to
- *                     K = 257, else 64)
+ *                     F32 on FP32 MFMA for K <= 513, by two fp16 terms where
+ *                     that is faster and up to K = 2049, by BF16x3 beyond
+ *                     (F32_EXACT as 2)
+ *   "direct.mfma_strip" 256-output tiles per wave of loader 3 (1 .. 4096; set,
+ *                     F32 stays on FP32 MFMA for K <= 513; default 4 for
+ *                     K <= 8, 8 to K = 40, 16 to K = 56, 32 to K = 257, else
+ *                     64, fewer on batches that would not fill the device)
  *   "direct.seg_tiles" tiles per workgroup of the pipelined direct kernel
  *   "direct.dma_bufs" LDS tile buffers of loader 2 (2, 3 or 4: 1 to 3 tiles in flight)
  *   "mfma.tiles"      32x32 output tiles per wave of the MFMA kernel (1, 2, 4)

@@ -409,7 +409,9 @@ extern "C" int scir_hip_autotune(const char *cache_path, int32_t budget_ms)
                 found.push_back(e);
             }
         }
-        // AUTO cut-over on long rows: the smallest K at which BF16x3 beats F32.
+        // AUTO cut-over on long rows: the smallest K at which BF16x3 beats F32
+        // on the FP32 matrix cores (a forced strip; by two fp16 terms F32 has a
+        // line of its own in AUTO, drawn by its error).
         int cut = TuneChoice{}.auto_mfma_min_k;
         if (status == SCIR_HIP_OK && !over_budget()) {
             {
@@ -423,6 +425,7 @@ extern "C" int scir_hip_autotune(const char *cache_path, int32_t budget_ms)
                 if (status != SCIR_HIP_OK) break;
                 const int64_t N = long_n, B = total / N;
                 float m32 = 0, m3 = 0;
+                set(-1, -1, -1, -1, -1, K <= 56 ? 16 : K <= 257 ? 32 : 64);
                 status = time_ms([&]() {
                     return scir_hip_fir_f32_dev(x, N, b, K, B, N, y, N, SCIR_HIP_PREC_F32, s);
                 }, s, 3, &m32);
@@ -435,6 +438,7 @@ extern "C" int scir_hip_autotune(const char *cache_path, int32_t budget_ms)
                     break;
                 }
             }
+            set(-1, -1, -1, -1, -1);
             if (cut < 0) cut = 1 << 20;
         }
         // FFT cut-over: the smallest K at which FP32 FFT beats BF16x3 MFMA.

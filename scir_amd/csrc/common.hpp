@@ -116,11 +116,13 @@ int fir_mfma_dev(const float *x, int64_t ldx, const float *b, int K, int64_t B, 
                  float *y, int64_t ldy, int precision, bool rev, hipStream_t stream,
                  DeviceState *st);
 // F32 by two fp16 terms (fir_f16x2.hip): whether it takes K taps (its LDS
-// leaves room for two workgroups a CU), and the filter itself, as_ragged in the
-// ragged kernel's segments (the samples' scale is a segment's: the same bits).
+// leaves room for two workgroups a CU), and the filter itself.  The segment
+// length goes by the whole batch's rows (the samples' scale is a segment's, so
+// it decides the bits); kRaggedRows gives the ragged kernel's.
+constexpr int64_t kRaggedRows = (int64_t)1 << 20;
 bool fir_f16x2_takes(int K);
 int fir_f16x2_dev(const float *x, int64_t ldx, const float *b, int K, int64_t B, int64_t N,
-                  float *y, int64_t ldy, bool rev, bool as_ragged, hipStream_t stream,
+                  float *y, int64_t ldy, bool rev, int64_t batch_rows, hipStream_t stream,
                   DeviceState *st);
 // Partial sums (floats) the allocation-free dL/db entry point holds: 4 MiB.
 constexpr size_t kVjpNoAllocPartials = (size_t)1 << 20;
@@ -129,9 +131,11 @@ int vjp_noalloc_scratch_address(void **ptr);
 
 // Whether the MFMA kernel's LDS holds K taps (one tile per wave).
 bool fir_mfma_takes(int precision, int K);
+// batch_rows: rows of the whole batch when B is a part of it (0: B), so that
+// every part runs by the whole batch's arithmetic.
 int fir_dense_dispatch(const float *x, int64_t ldx, const float *b, int32_t K, int64_t B,
                        int64_t N, float *y, int64_t ldy, int32_t precision, bool rev,
-                       hipStream_t stream, DeviceState *st);
+                       hipStream_t stream, DeviceState *st, int64_t batch_rows = 0);
 int fill_zero_2d(float *y, int64_t ldy, int64_t B, int64_t N, hipStream_t stream);
 
 // ---- ragged (CSR) batches on MFMA ----------------------------------------

@@ -598,10 +598,11 @@ int fir_direct_dev(const float *x, int64_t ldx, const float *b, int K, int64_t B
         // and 129: [1, 262144] 5.3 -> 3.0 us and 35 -> 4.3, [64, 16384] 5.8 ->
         // 4.1 and 35 -> 6.7; [64, 65536] 8.1 and 36 -> 16), evened out over
         // the row.
+        // (A tuned table's strips come from a large batch: the same holds.)
         int64_t strip = tc.direct_mfma_strip;
-        if (strip <= 0) {
+        if (strip <= 0) strip = K <= 8 ? 4 : K <= 40 ? 8 : K <= 56 ? 16 : K <= 257 ? 32 : 64;
+        if (!tc.direct_mfma_strip_forced) {
             const int64_t row_tiles = (N + kMfmaTile - 1) / kMfmaTile, tiles = B * row_tiles;
-            strip = K <= 8 ? 4 : K <= 40 ? 8 : K <= 56 ? 16 : K <= 257 ? 32 : 64;
             const int64_t fill =
                 std::max(std::min<int64_t>((tiles + 1024) / 2048, 2), (tiles + 2048) / 4096);
             strip = std::max<int64_t>(1, std::min({strip, fill, row_tiles}));
@@ -692,12 +693,13 @@ bool takes_bf16x3(const TuneChoice &tc, int K, int64_t B, int64_t N)
 
 // The F32 mode.
 int fir_f32_dev(const float *x, int64_t ldx, const float *b, int K, int64_t B, int64_t N,
-                float *y, int64_t ldy, bool rev, hipStream_t stream, DeviceState *st)
+                float *y, int64_t ldy, bool rev, hipStream_t stream, DeviceState *st,
+                int64_t batch_rows)
 {
     const TuneChoice tc = tune_lookup(K, N);
-    if (takes_f16x2(tc, K, B, N))
-        return fir_f16x2_dev(x, ldx, b, K, B, N, y, ldy, rev, false, stream, st);
-    if (takes_bf16x3(tc, K, B, N))
+    if (takes_f16x2(tc, K, batch_rows, N))
+        return fir_f16x2_dev(x, ldx, b, K, B, N, y, ldy, rev, batch_rows, stream, st);
+    if (takes_bf16x3(tc, K, batch_rows, N))
         return fir_mfma_dev(x, ldx, b, K, B, N, y, ldy, SCIR_HIP_PREC_BF16X3, rev, stream, st);
     return fir_direct_dev(x, ldx, b, K, B, N, y, ldy, false, rev, stream, st);
 }
@@ -708,11 +710,12 @@ int fir_f32_dev(const float *x, int64_t ldx, const float *b, int K, int64_t B, i
 // adjoint (rev = true: the same filter run back to front).
 int fir_dense_dispatch(const float *x, int64_t ldx, const float *b, int32_t K, int64_t B,
                        int64_t N, float *y, int64_t ldy, int32_t precision, bool rev,
-                       hipStream_t stream, DeviceState *st)
+                       hipStream_t stream, DeviceState *st, int64_t batch_rows)
 {
+    if (batch_rows == 0) batch_rows = B;
     switch (precision) {
     case SCIR_HIP_PREC_F32:
-        return fir_f32_dev(x, ldx, b, K, B, N, y, ldy, rev, stream, st);
+        return fir_f32_dev(x, ldx, b, K, B, N, y, ldy, rev, stream, st, batch_rows);
     case SCIR_HIP_PREC_F32_EXACT:
         return fir_direct_dev(x, ldx, b, K, B, N, y, ldy, true, rev, stream, st);
     case SCIR_HIP_PREC_BF16X3:
@@ -726,9 +729,9 @@ int fir_dense_dispatch(const float *x, int64_t ldx, const float *b, int32_t K, i
             return fir_fft_dev(x, ldx, b, K, B, N, y, ldy, rev, stream, st);
         // BF16x3 MFMA from the cut-over up, while its LDS holds the taps.
         if (K >= tc.auto_mfma_min_k && fir_mfma_takes(SCIR_HIP_PREC_BF16X3, K) &&
-            !auto_takes_f16x2(tc, K, B, N))
+            !auto_takes_f16x2(tc, K, batch_rows, N))
             return fir_mfma_dev(x, ldx, b, K, B, N, y, ldy, SCIR_HIP_PREC_BF16X3, rev, stream, st);
-        return fir_f32_dev(x, ldx, b, K, B, N, y, ldy, rev, stream, st);
+        return fir_f32_dev(x, ldx, b, K, B, N, y, ldy, rev, stream, st, batch_rows);
     }
     default:
         return fail(SCIR_HIP_ERR_INVALID_ARGUMENT, "unknown precision %d", precision);
@@ -1028,7 +1031,7 @@ int host_fir_pipelined(const float *x, int64_t ldx, const float *db, int32_t K, 
             break;
         }
         const int st2 = fir_dense_dispatch(dx + r0 * ldd, ldd, db, K, rows_of(c), N,
-                                           dy + r0 * ldd, ldd, precision, false, sk, st);
+                                           dy + r0 * ldd, ldd, precision, false, sk, st, B);
         if (st2 != SCIR_HIP_OK) {
             pipe.fail_with(st2, scir_hip_last_error());
             break;

@@ -490,7 +490,7 @@ bool fir_f16x2_takes(int K)
 }
 
 int fir_f16x2_dev(const float *x, int64_t ldx, const float *b, int K, int64_t B, int64_t N,
-                  float *y, int64_t ldy, bool rev, bool as_ragged, hipStream_t stream,
+                  float *y, int64_t ldy, bool rev, int64_t batch_rows, hipStream_t stream,
                   DeviceState *st)
 {
     if (B == 0 || N == 0) return SCIR_HIP_OK;
@@ -499,8 +499,8 @@ int fir_f16x2_dev(const float *x, int64_t ldx, const float *b, int K, int64_t B,
     // Segments of 8192 samples once two workgroups a CU have one ([64, 65536],
     // K = 129: 14.2 us against 17.0 with 4096), of 4096 for fewer or shorter
     // rows ([64, 16384], K = 512: 10.2 against 12.8).
-    const int64_t long_segs = B * ((N + kMfmaRaggedSegLen - 1) / kMfmaRaggedSegLen);
-    const int tw = N <= 4096 || (!as_ragged && long_segs < 2 * (int64_t)st->cu_count) ? 1 : 2;
+    const int64_t long_segs = batch_rows * ((N + kMfmaRaggedSegLen - 1) / kMfmaRaggedSegLen);
+    const int tw = N <= 4096 || long_segs < 2 * (int64_t)st->cu_count ? 1 : 2;
     const int64_t seg_len = 32 * (int64_t)kWaves * tw * 32;
     const int64_t total = B * ((N + seg_len - 1) / seg_len);
     const int64_t cap = tc.mfma_segs_forced

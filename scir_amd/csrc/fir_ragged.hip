@@ -295,7 +295,7 @@ int scir_hip_ragged_plan_execute_per_signal(scir_hip_ragged_plan plan, const flo
             if (len == 0) continue;
             if (plan->split)
                 SCIR_TRY(fir_f16x2_dev(x + plan->offs[i], len, b + plan->boffs[i], K, 1, len,
-                                       y + plan->offs[i], len, false, true, s, st));
+                                       y + plan->offs[i], len, false, kRaggedRows, s, st));
             else if (mode == kMfma)
                 SCIR_TRY(fir_mfma_dev(x + plan->offs[i], len, b + plan->boffs[i], K, 1, len,
                                       y + plan->offs[i], len, plan->precision, false, s, st));

@@ -127,6 +127,29 @@ def test_taken_from_its_size_up_matches_fp32_matrix_cores(hip, oracle):
     assert np.all(np.abs(y - y64) <= lim) and np.all(np.abs(y32 - y64) <= lim)
 
 
+@pytest.mark.parametrize("K,precision", [(1023, "f32"), (300, "auto"), (2100, "f32")])
+def test_parts_of_a_batch_run_by_its_arithmetic(hip, K, precision):
+    """A batch that the host tier takes in parts of one row: the bits of the
+    whole on the device, where a row by itself would run another way."""
+    import torch
+    from scir_amd import device
+    L = hip.lib()
+    r = rng(K)
+    x = r.standard_normal((70, 65536)).astype(np.float32)
+    b = r.standard_normal(K).astype(np.float32)
+    print(f"f16x2 parts {precision} K={K}", flush=True)
+    want = device.fir(torch.tensor(x, device="cuda"), torch.tensor(b, device="cuda"), precision)
+    y = np.empty_like(x)
+    hip.check(L.scir_hip_tune_set(b"host.chunk_kib", 256))
+    try:
+        hip.check(L.scir_hip_fir_f32_host(
+            x.ctypes.data, x.shape[1], b.ctypes.data, K, *x.shape, y.ctypes.data, x.shape[1],
+            hip.precision_code(precision)))
+    finally:
+        hip.check(L.scir_hip_tune_set(b"host.chunk_kib", -1))
+    assert np.array_equal(y, want.cpu().numpy())
+
+
 def test_long_segments_of_many_rows(hip, oracle):
     """Rows enough that the segments are of 8192 samples (test_segment_edges
     has the short ones): one, and one sample into the second."""
