@@ -29,27 +29,24 @@ __global__ __launch_bounds__(kThreads) void fir_mfma_kernel(
     constexpr int PF = 2 * TW + 1;
     const int64_t lid = xcd_remap(blockIdx.x, nwg);
     const int64_t seg_first = lid * segs_per_wg;
-    const int64_t seg_end = min(nsegs, seg_first + segs_per_wg);
+    const int count = (int)min((int64_t)segs_per_wg, nsegs - seg_first);
     const int units = SEG_BLOCKS * 4 + 2 * m_hi;
-
-    // Row pointer and sample index of LDS unit 0 of segment sg.
-    auto seg_base = [&](int64_t sg, const float *&xrow, int64_t &xb, int64_t &P0, int64_t &row) {
-        row = row0 + sg / segs_per_row;
-        P0 = (sg % segs_per_row) * SEG_BLOCKS;
-        xrow = x + row * ldx;
-        xb = 32 * P0 - 16 * (int64_t)m_hi;
-    };
+    // Row and segment of the row, stepped: a 64-bit division is some 150
+    // scalar instructions, and one stood before every contraction.
+    const int64_t first_row = seg_first / segs_per_row;
+    int seg = (int)(seg_first - first_row * segs_per_row);
+    const float *xrow = x + (row0 + first_row) * ldx;
+    float *yrow = y + (row0 + first_row) * ldy;
 
     f32x4 raw[PF][2];
-    auto prefetch = [&](int64_t sg, int tid) {
-        const float *xrow;
-        int64_t xb, P0, row;
-        seg_base(sg, xrow, xb, P0, row);
+    // Sample index of LDS unit 0 of a row's segment sg.
+    auto first_sample = [&](int sg) { return 32 * (int64_t)sg * SEG_BLOCKS - 16 * (int64_t)m_hi; };
+    auto prefetch = [&](const float *xr, int sg, int tid) {
 #pragma unroll
         for (int j = 0; j < PF; ++j)
-            load_unit<REV>(xrow, N, xb, tid + j * kThreads, units, raw[j]);
+            load_unit<REV>(xr, N, first_sample(sg), tid + j * kThreads, units, raw[j]);
     };
-    prefetch(seg_first, (int)threadIdx.x);
+    prefetch(xrow, seg, (int)threadIdx.x);
 
     // Tap tables, built while the first segment's loads are in flight.
     int *mins = reinterpret_cast<int *>(lds + tab_offset + 2 * S * copy_bytes);
@@ -62,7 +59,7 @@ __global__ __launch_bounds__(kThreads) void fir_mfma_kernel(
         }
     }
 
-    for (int64_t sg = seg_first; sg < seg_end; ++sg) {
+    for (int done = 0; done < count; ++done) {
         // Lane-dependent values are recomputed in every iteration rather than
         // hoisted out of the loop, where they would hold registers through
         // the contraction.
@@ -70,12 +67,12 @@ __global__ __launch_bounds__(kThreads) void fir_mfma_kernel(
         asm volatile("" : "+v"(tid));
         const int wave = tid >> 6, lane = tid & 63;
         const int i = lane & 31, g = lane >> 5;
-        const float *xrow;
-        int64_t xb, P0, row;
-        seg_base(sg, xrow, xb, P0, row);
+        const int64_t P0 = (int64_t)seg * SEG_BLOCKS, xb = first_sample(seg);
+        const bool last = seg + 1 == segs_per_row;
+        const int next_seg = last ? 0 : seg + 1;
 
         // ---- stage: x[xb .. xb + 8*units) -> S split arrays in LDS ----
-        if (sg != seg_first) __syncthreads();  // the previous segment's MFMAs are done
+        if (done) __syncthreads();  // the previous segment's MFMAs are done
         int min_e = 0;
         stage_segment<S, TW, PF, REV>(lds, split_stride, raw, xrow, N, xb, units, tid, min_e);
         if (S == 3) {
@@ -83,7 +80,7 @@ __global__ __launch_bounds__(kThreads) void fir_mfma_kernel(
             if (lane == 0) mins[wave] = m;
         }
         __syncthreads();
-        if (sg + 1 < seg_end) prefetch(sg + 1, tid);
+        if (done + 1 < count) prefetch(last ? xrow + ldx : xrow, next_seg, tid);
 
         // ---- contraction and epilogue ----
         // Wave w's tiles cover outputs 32*(P0 + 32*TW*w) .. +1024*TW-1 of the
@@ -98,7 +95,12 @@ __global__ __launch_bounds__(kThreads) void fir_mfma_kernel(
             // Read after the contraction (the words change only after the
             // next segment's first barrier): nothing extra stays live through it.
             const bool tiny = S == 3 && segment_is_tiny(mins);
-            store_segment<S, TW, REV>(ct, y + row * ldy, N, P0, wave, i, g, xrow, b, K, tiny);
+            store_segment<S, TW, REV>(ct, yrow, N, P0, wave, i, g, xrow, b, K, tiny);
+        }
+        seg = next_seg;
+        if (last) {
+            xrow += ldx;
+            yrow += ldy;
         }
     }
 }

@@ -374,7 +374,10 @@ struct Contraction {
         // rest as unrolled RS-iteration bodies with no branches.
         body<P, 0, kFirst>(0, count);
         int n0 = RS;
-        for (; n0 + RS <= count; n0 += RS) body<P, 0, kPlain>(n0, count);
+        for (; n0 + RS <= count; n0 += RS) {
+            if (S == 3 && 2 * n0 >= count) __builtin_amdgcn_s_setprio(1);
+            body<P, 0, kPlain>(n0, count);
+        }
         // At most RS - 1 + (2TW - 2) < 2*RS iterations remain.
         tail<P, 0>(n0, count);
         tail<P, 0>(n0 + RS, count);
@@ -392,11 +395,12 @@ struct Contraction {
     __device__ __forceinline__ void run()
     {
         const int half = CH == 2 ? msteps / 2 : msteps;  // msteps >= 2
-        // Two passes: of the two waves on a SIMD, the one that is further on
-        // goes first, up to its next contraction.  Equal shares keep the two
-        // in step, and staging and stores of both then meet (K = 512: 1780 ->
-        // 1733 us, 1023: 374 -> 355).
-        if constexpr (CH == 2) __builtin_amdgcn_s_setprio(0);
+        // Of the two waves on a SIMD, the one in the second half of its
+        // half-steps goes first, up to its next contraction.  Equal shares
+        // keep the two in step, and staging and stores of both then meet
+        // (F16x2, K = 512: 1780 -> 1733 us, 1023: 374 -> 355; BF16x3 with its
+        // row index stepped, K = 512: 2655 -> 2540).
+        if constexpr (S > 1) __builtin_amdgcn_s_setprio(0);
         pass<0>(half);
         if constexpr (CH == 2) {
             __builtin_amdgcn_s_setprio(1);
