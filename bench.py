@@ -11,12 +11,11 @@ in HBM.  ``value`` = output samples / second over the K timed steps (device
 time, HIP events on the launch stream).  Beside it the line carries, measured
 after the timed region on the same inputs:
   compare.f32 / compare.fp16         the other arithmetic paths, Gsamples/s
-  / compare.fft32                     (f32: FP32, on the FP32 matrix cores up to
-                                      K = 513; fft32: FP32 FFT overlap-save,
+  / compare.fft32                     (f32: FP32, by two fp16 terms on the 16-bit
+                                      matrix cores here; fft32: FP32 FFT overlap-save,
                                       normwise error) and rel-L2 vs the FP64 oracle
   compare.fp32_direct_valu            the FP32 direct form on the vector units
-                                      (fused multiply-adds; what F32 runs above
-                                      K = 513)
+                                      (fused multiply-adds)
   bandwidth_workload                  x [4096, 65536], 33-tap low-pass, FP32:
                                       GB/s against the 8 TB/s HBM peak
   roofline                            the dominant kernel of the headline:
@@ -57,6 +56,9 @@ HBM_PEAK_GBS = 8000.0
 BF16_PEAK_TFLOPS = 2500.0   # dense bf16/fp16 MFMA, MI355X
 FP32_PEAK_TFLOPS = 157.3
 F32_MFMA_MAX_K = 513  # the F32 mode's FP32-MFMA kernel takes K up to here
+# On long rows F32 runs by two fp16 terms (fir_f16x2_kernel) from here up to the
+# second, BF16x3 beyond.
+F32_SPLIT_MIN_K, F32_SPLIT_MAX_K = 97, 2049
 
 METRIC = "FIR Gsamples/s & %roofline: bf16x3 MFMA vs FP32 direct at rel L2 err<=1e-6"
 
@@ -306,7 +308,22 @@ def roofline_for(wl, name, prec, avg_launch_s):
                     ceiling_note=f"{prods} MFMA products x {mfma_steps(wl['K'])} half-steps of "
                                  "32x32x16 per 32x32 output tile at 2.5 PFLOP/s")
     flops = 2.0 * wl["K"] * samples
-    # F32 up to K = 513 runs on the FP32 matrix cores (a 16 x 16(NG) Toeplitz
+    if prec == "f32" and F32_SPLIT_MIN_K <= wl["K"] <= F32_SPLIT_MAX_K:
+        # Three 16-bit products a tap: HBM-bound until they outweigh 8 B a sample.
+        issued = 32.0 * mfma_steps(wl["K"]) * 3 * samples
+        extra = dict(kernel="fir_f16x2_kernel (two fp16 terms, v_mfma_f32_32x32x16_f16)",
+                     mfma_issued_tflops=round(issued / avg_launch_s / 1e12, 1),
+                     mfma_issued_frac=round(issued / avg_launch_s / 1e12 / BF16_PEAK_TFLOPS, 4))
+        if issued / (BF16_PEAK_TFLOPS * 1e12) < 8.0 * samples / (HBM_PEAK_GBS * 1e9):
+            ach = 8.0 * samples / avg_launch_s / 1e9
+            return dict(bound="hbm", achieved=round(ach, 1), peak=HBM_PEAK_GBS, unit="GB/s",
+                        frac=round(ach / HBM_PEAK_GBS, 4),
+                        traffic=load_traffic(f"fir_f16x2_{name}_pmc"), **extra)
+        ach = flops / avg_launch_s / 1e12
+        return dict(bound="mfma", achieved=round(ach, 2), peak=BF16_PEAK_TFLOPS, unit="TFLOP/s",
+                    frac=round(ach / BF16_PEAK_TFLOPS, 4),
+                    traffic=load_traffic(f"fir_f16x2_{name}_pmc"), **extra)
+    # F32 on shorter filters runs on the FP32 matrix cores (a 16 x 16(NG) Toeplitz
     # block per 256 outputs, NG = ceil((K-1)/16) + 1); FP32 MFMA and FP32
     # vector share the 157.3 TFLOP/s peak on MI355X.
     f32_mfma = prec == "f32" and wl["K"] <= F32_MFMA_MAX_K
@@ -370,11 +387,12 @@ def run_dense(args):
                 rel_l2_vs_fp64=rel_l2_rows(x, y, b_np, rows))
             if other == "f32":
                 comp[other]["kernel"] = ("fir_direct_mfma_kernel (FP32 MFMA)"
-                                         if K <= F32_MFMA_MAX_K else "fir_direct_dma_kernel (FP32 VALU)")
+                                         if K < F32_SPLIT_MIN_K else
+                                         "fir_f16x2_kernel (two fp16 terms on MFMA)"
+                                         if K <= F32_SPLIT_MAX_K else
+                                         "fir_mfma_kernel (BF16x3 MFMA)")
         # The FP32 direct form on the VALU (fused multiply-adds, the LDS-DMA
-        # loader), which F32 runs only above K = 513; below, F32 runs on the
-        # FP32 matrix cores and this is the same arithmetic class timed on
-        # the vector units.
+        # loader): the same arithmetic class timed on the vector units.
         if K <= F32_MFMA_MAX_K:
             from scir_amd import _lib
             _lib.check(_lib.lib().scir_hip_tune_set(b"direct.loader", 2))
@@ -589,7 +607,8 @@ def run_ragged(args):
 def vjp_results(steps, warmup, prec, stream):
     """Forward + dL/dx + dL/db for x [1024, 65536], K = 255 low-pass,
     L = sum(w * y): Gsamples/s of the whole step, and the dL/db kernel
-    (FP32 MFMA) against the FP32 MFMA peak."""
+    against the peak of the 16-bit matrix cores that it runs on (four products
+    a multiply-add)."""
     import torch
     from scir_amd import design, device
     B, N, K = 1024, 65536, 255
@@ -611,12 +630,12 @@ def vjp_results(steps, warmup, prec, stream):
                 precision=prec, gsamples_s=round(B * N / (ms * 1e-3) / 1e9, 2),
                 ms_per_step=round(ms, 4), wall_s=round(wall, 3),
                 db_ms=round(ms_db, 4),
-                roofline=dict(bound="fp32", achieved=round(ach, 2), peak=FP32_PEAK_TFLOPS,
-                              unit="TFLOP/s", frac=round(ach / FP32_PEAK_TFLOPS, 4),
-                              kernel="fir_vjp_db_mfma_kernel (FP32 MFMA)",
-                              traffic=load_traffic(f"fir_vjp_db_{prec}_vjp_k255_pmc"),
-                              mfma_busy_frac=load_profile(f"fir_vjp_db_{prec}_vjp_k255_util",
-                                                          "mfma_busy_frac")))
+                roofline=dict(bound="mfma", achieved=round(ach, 2), peak=BF16_PEAK_TFLOPS,
+                              unit="TFLOP/s", frac=round(ach / BF16_PEAK_TFLOPS, 4),
+                              kernel="fir_vjp_db_split_kernel (two fp16 terms on MFMA)",
+                              mfma_issued_tflops=round(4 * 2.0 * 256 * B * N
+                                                       / (ms_db * 1e-3) / 1e12, 1),
+                              traffic=load_traffic(f"fir_vjp_db_split_{prec}_vjp_k255_pmc")))
 
 
 def run_vjp(args):

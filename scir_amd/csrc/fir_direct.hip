@@ -645,7 +645,7 @@ namespace {
 // F32 by two fp16 terms (fir_f16x2.hip).
 //   * Above 513 taps, the end of the FP32 matrix-core kernel, always: the VALU
 //     form it replaces is slower at every size ([1, 5000], K = 1023: 21.3 ->
-//     17.0 us; [1024, 65536], K = 1023: 1810 -> 378 us).
+//     12.6 us; [1024, 65536], K = 1023: 1810 -> 350 us).
 //   * Up to 513 the two cost about staged * (27 + ng) against c * outputs * ng
 //     (staged: whole segments; ng: groups of 16 taps), c = 5 up to K = 257 and
 //     8 above, where the FP32 kernel needs a second tile of history.  They
@@ -666,8 +666,8 @@ bool takes_f16x2(const TuneChoice &tc, int K, int64_t B, int64_t N)
 }
 
 // AUTO chooses between BF16x3 and F32 from its cut-over up.  By two fp16 terms
-// F32 is the faster from there ([4096, 65536], K = 200: 610 against 765 us;
-// [2048, 262144], K = 512: 1830 against 2630), but only from here is its error
+// F32 is the faster from there ([4096, 65536], K = 200: 600 against 730 us;
+// [2048, 262144], K = 512: 1733 against 2540), but only from here is its error
 // no larger for any of 34 filters and inputs (relative L2 against BF16x3's:
 // 0.82 on average and 0.95 at most at K = 300, 0.68 and 0.82 at 512; 0.85 and
 // 1.05 at 255, 1.08 and 1.32 at 129), and small batches lose its longer start

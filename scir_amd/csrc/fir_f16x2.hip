@@ -12,14 +12,15 @@
 //
 // Measured, us a call (before: the FP32 matrix cores to K = 513, the VALU
 // above; in brackets BF16x3):
-//   [4096, 65536]   K = 129   698 -> 540  (620)    255  1274 -> 655  (835)
-//   [2048, 262144]  K = 512  5550 -> 1830 (2640)  2048 28700 -> 5060 (8640)
-//   [1024, 65536]   K = 1023 1818 -> 378
-//   2500 ragged signals, K 15 .. 1023: 4370 -> 1110 (1625)
-// At K = 512 the matrix cores are busy 57 % of the cycles at a clock that the
-// load pulls down to about 1.6 GHz, so the bound is power and the phases that
-// do not overlap (staging and stores of one wave against the contraction of
-// the other on its SIMD); below K = 200 it is those phases alone.
+//   [4096, 65536]   K = 129   698 -> 515  (600)    255  1274 -> 612  (810)
+//   [2048, 262144]  K = 512  5550 -> 1733 (2540)
+//   [1024, 65536]   K = 1023 1818 -> 350  (600)   2040  3572 -> 610 (1060)
+//   2500 ragged signals, K 15 .. 1023: 4370 -> 1080 (1625)
+// At K = 512 the matrix cores are busy 61 % of the cycles at a clock that the
+// load pulls down to 1.4 GHz (with one workgroup a CU it runs at 1.9), so the
+// bound is power; below K = 200 it is HBM and the phases that do not overlap
+// (staging and stores of one wave against the contraction of the other on its
+// SIMD).
 //
 // Range.  fp16 has five exponent bits, so samples and taps are scaled by
 // powers of two: the taps by 2^sb, which puts the largest in [2^13, 2^14), the
