@@ -329,8 +329,9 @@ __device__ __forceinline__ void group_span(int64_t gidx, int64_t ngroups, int64_
 }
 
 // A lane's group from zero state, in time order: outputs in place of the
-// samples, end state in s1, s2.  (The wave kernel's own direction has the same
-// in line: called, its loop took 939 us instead of 934 on [4096, 65536].)
+// samples, end state in s1, s2.  (The state and run kernels have it in line:
+// with the call the run took 939 us instead of 934 on [4096, 65536], while the
+// collecting kernel of three sections spills without.)
 template <int SMAX, bool REV>
 __device__ __forceinline__ void filter_group(double (&v)[kGroup], int64_t cnt, bool all_full,
                                              double (&s1)[SMAX], double (&s2)[SMAX],
@@ -505,27 +506,31 @@ sos_wave_kernel(
         } else {
             load_lane(v, xr, lo, cnt, vb);
         }
-        // The lane's samples from zero state, in time order (filter_group).
+        // The lane's samples from zero state, in time order.
         double s1[SMAX], s2[SMAX];
+        if constexpr (MODE == kCollect) {
+            filter_group<SMAX, REV>(v, cnt, __all(full), s1, s2, cf, S);
+        } else {  // the same in line (see there)
 #pragma unroll
-        for (int i = 0; i < SMAX; ++i) s1[i] = s2[i] = 0.0;
-        if (__all(full)) {
-            if (!REV) {
+            for (int i = 0; i < SMAX; ++i) s1[i] = s2[i] = 0.0;
+            if (__all(full)) {
+                if (!REV) {
 #pragma unroll
-                for (int k = 0; k < kGroup; ++k) v[k] = df2t_step<SMAX>(v[k], s1, s2, cf, S);
+                    for (int k = 0; k < kGroup; ++k) v[k] = df2t_step<SMAX>(v[k], s1, s2, cf, S);
+                } else {
+#pragma unroll
+                    for (int k = kGroup - 1; k >= 0; --k) v[k] = df2t_step<SMAX>(v[k], s1, s2, cf, S);
+                }
             } else {
+                if (!REV) {
 #pragma unroll
-                for (int k = kGroup - 1; k >= 0; --k) v[k] = df2t_step<SMAX>(v[k], s1, s2, cf, S);
-            }
-        } else {
-            if (!REV) {
+                    for (int k = 0; k < kGroup; ++k)
+                        if (k < cnt) v[k] = df2t_step<SMAX>(v[k], s1, s2, cf, S);
+                } else {
 #pragma unroll
-                for (int k = 0; k < kGroup; ++k)
-                    if (k < cnt) v[k] = df2t_step<SMAX>(v[k], s1, s2, cf, S);
-            } else {
-#pragma unroll
-                for (int k = kGroup - 1; k >= 0; --k)
-                    if (k < cnt) v[k] = df2t_step<SMAX>(v[k], s1, s2, cf, S);
+                    for (int k = kGroup - 1; k >= 0; --k)
+                        if (k < cnt) v[k] = df2t_step<SMAX>(v[k], s1, s2, cf, S);
+                }
             }
         }
         double e[D];
