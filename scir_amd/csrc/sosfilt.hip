@@ -926,6 +926,14 @@ int sos_run(const double *x, int64_t ldx, double *y, int64_t ldy, int64_t rows, 
     }
     SosPlan p{};
     sos_plan(rows, N, st->cu_count, reference_order, &p.row_mode, &p.L, &p.nC);
+    // Chunks of two steps where twice as many of one could not be collected
+    // ([14, 262000], order 4: 38 -> 31 us, filtfilt 71 -> 58; a single row of
+    // four sections gains nothing, 47.1 -> 48.4).
+    if (p.nC > kMaxChunks && p.L == kStep && N <= kMaxChunks * 2 * kStep && S <= kCollectMaxS &&
+        (S < kCollectMaxS || rows > 1)) {
+        p.L = 2 * kStep;
+        p.nC = (N + p.L - 1) / p.L;
+    }
     if ((p.row_mode ? rows : rows * p.nC / (kThreads / 64)) + 2 > 0x7fffffffLL)
         return fail(SCIR_HIP_ERR_INVALID_ARGUMENT, "too many rows");
     if (!p.row_mode) {
